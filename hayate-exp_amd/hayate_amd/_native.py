@@ -94,6 +94,14 @@ _SIGNATURES = {
         [_P, _I64, _I64, _I64, _P, _P, _I32, _I32, _P, _I64, _I32, _I32, _I32, _P],
         ctypes.c_int,
     ),
+    "hy_norm_linear": (
+        [_P, _I64, _I32, _I32, _P, _F32, _P, _P, _I64, _I32, _P, _I64, _P],
+        ctypes.c_int,
+    ),
+    "hy_linear_add": (
+        [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _I64, _P, _I64, _P],
+        ctypes.c_int,
+    ),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)

@@ -92,10 +92,13 @@ class GroupedQueryAttention(nn.Module):
     def project_qkv(self, x):
         """x (B, T, d_in) -> q (B, T, Hq, D), k, v (B, T, Hkv, D): strided views
         of one GEMM output (row stride (Hq + 2 Hkv) * D)."""
-        B, T, _ = x.shape
+        return self.split_qkv(F.linear(x, self.fused_qkv_weight()))
+
+    def split_qkv(self, y):
+        """The q, k and v views of a fused projection's output (B, T, rows)."""
+        B, T, _ = y.shape
         hq = self.num_heads * self.head_dim
         hkv = self.num_kv_groups * self.head_dim
-        y = F.linear(x, self.fused_qkv_weight())
         q = y[..., :hq].view(B, T, self.num_heads, self.head_dim)
         k = y[..., hq : hq + hkv].view(B, T, self.num_kv_groups, self.head_dim)
         v = y[..., hq + hkv :].view(B, T, self.num_kv_groups, self.head_dim)
@@ -122,8 +125,13 @@ class GroupedQueryAttention(nn.Module):
             raise NotImplementedError(
                 "only the paged attention path is provided (pass paged_cache)"
             )
-        B, T, _ = x.shape
-        q, k, v = self.project_qkv(x)
+        context = self.context(*self.project_qkv(x), cos, sin, paged_cache, layer_idx)
+        return self.o_proj(context), None, None
+
+    def context(self, q, k, v, cos, sin, paged_cache, layer_idx):
+        """Norm, rope, append and paged attention of projected q, k, v (B, T,
+        H, D): the input of o_proj, (B, T, Hq * D)."""
+        B, T = q.shape[:2]
         q_norm_w = self.q_norm.weight
         k_norm_w = self.k_norm.weight
         # each norm keeps its own eps; None means the input dtype's epsilon,
@@ -157,5 +165,4 @@ class GroupedQueryAttention(nn.Module):
                 layer_idx, q, k, v, q_norm_w, k_norm_w, eps, cos, sin, k_eps=k_eps
             )
             context = paged_cache.attend_layer(q_rot.transpose(1, 2), layer_idx).transpose(1, 2)
-        context = context.reshape(B, T, self.num_heads * self.head_dim)
-        return self.o_proj(context), None, None
+        return context.reshape(B, T, self.num_heads * self.head_dim)

@@ -1,0 +1,122 @@
+"""The products of a decode tick's few rows with the model's weights
+(csrc/skinny.hip), and the rule that says when a module's forward may take
+them in place of its submodules' own calls.
+
+``norm_linear`` is RMSNorm then a projection (optionally the gated pair with
+silu), ``linear_add`` a projection plus the residual. They compute what the
+torch modules do with fp32 sums and fewer bf16 roundings, and know nothing of
+autograd, hooks or tracing: ``few_rows`` and ``plain`` hold every condition
+under which a caller must leave the modules in charge.
+"""
+
+from __future__ import annotations
+
+from typing import Optional
+
+import torch
+import torch.nn as nn
+from torch.nn.modules import module as _module
+
+from . import _native
+
+MAX_ROWS = 32
+
+
+def few_rows(x: torch.Tensor) -> bool:
+    """True when `x` (..., d) is a plain bf16 tensor of at most MAX_ROWS rows on
+    the current HIP device and nothing watches the operators run on it
+    (gradients, autocast, tracing, dispatch or function modes, functorch)."""
+    if (type(x) is not torch.Tensor or x.dtype is not torch.bfloat16 or not x.is_cuda
+            or not 0 < x.numel() <= MAX_ROWS * x.shape[-1]
+            or torch.is_grad_enabled() or torch.is_autocast_enabled()):
+        return False
+    c = torch._C
+    return (c._len_torch_dispatch_stack() == 0 and c._len_torch_function_stack() == 0
+            and c._get_tracing_state() is None and not torch.compiler.is_compiling()
+            and torch.autograd.forward_ad._current_level < 0
+            and c._functorch.peek_interpreter_stack() is None
+            and x.device.index == torch.cuda.current_device())
+
+
+def _bare(m: nn.Module) -> bool:
+    """No hooks and no forward of its own."""
+    d = m.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                or d["_backward_pre_hooks"] or "forward" in d)
+
+
+def _plain_weight(w, like: torch.Tensor, dim: int) -> bool:
+    return (type(w) is nn.Parameter and w.dtype is torch.bfloat16 and w.device == like.device
+            and w.dim() == dim and w.stride(-1) == 1 and w.data_ptr() & 15 == 0
+            and (dim == 1 or w.stride(0) & 7 == 0))
+
+
+def plain(x: torch.Tensor, modules=(), norms=(), linears=()) -> bool:
+    """True when calling `modules`, `norms` (over x's last dimension) and
+    `linears` would do nothing but their own arithmetic on weights that the
+    kernels can read."""
+    if _module._has_any_global_hook():
+        return False
+    for m in modules:
+        if not _bare(m):
+            return False
+    for m in norms:
+        if not (type(m) is nn.RMSNorm and _bare(m) and m.normalized_shape == (x.shape[-1],)
+                and _plain_weight(m._parameters.get("weight"), x, 1)):
+            return False
+    for m in linears:
+        if not (type(m) is nn.Linear and _bare(m) and m._parameters.get("bias") is None
+                and _plain_weight(m._parameters.get("weight"), x, 2)):
+            return False
+    return True
+
+
+def norm_fits(k: int, rows: int) -> bool:
+    """Sizes hy_norm_linear takes."""
+    return k % 64 == 0 and 512 <= k <= 4096 and rows <= (MAX_ROWS if k <= 3072 else 16)
+
+
+def add_fits(k: int, rows: int) -> bool:
+    """Sizes hy_linear_add takes."""
+    return k % 128 == 0 and k > 0 and rows <= MAX_ROWS
+
+
+def rows_of(x: torch.Tensor) -> torch.Tensor:
+    """x (..., d) as (rows, d) with rows the kernels can read."""
+    x = x.reshape(-1, x.shape[-1])
+    if x.stride(1) != 1 or x.stride(0) & 7 or x.data_ptr() & 15:
+        x = x.contiguous()
+        if x.data_ptr() & 15:
+            x = x.clone()
+    return x
+
+
+def norm_linear(x: torch.Tensor, norm_weight: Optional[torch.Tensor], eps: float,
+                weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """norm(x) W^T, or silu(norm(x) W^T) * (norm(x) U^T); x is (rows, k)."""
+    m, k = x.shape
+    n = weight.shape[0]
+    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    rc = _native.lib().hy_norm_linear(
+        x.data_ptr(), x.stride(0), m, k, None if norm_weight is None else norm_weight.data_ptr(),
+        eps, weight.data_ptr(), None if up_weight is None else up_weight.data_ptr(),
+        weight.stride(0), n, y.data_ptr(), n, torch.cuda.current_stream(x.device).cuda_stream)
+    if rc:
+        _native.check(rc, "hy_norm_linear")
+    return y
+
+
+def linear_add(x: torch.Tensor, weight: torch.Tensor,
+               residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x W^T + residual; x is (rows, k)."""
+    m, k = x.shape
+    n = weight.shape[0]
+    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    rc = _native.lib().hy_linear_add(
+        x.data_ptr(), x.stride(0), m, k, weight.data_ptr(), weight.stride(0), n,
+        None if residual is None else residual.data_ptr(),
+        0 if residual is None else residual.stride(0), y.data_ptr(), n,
+        torch.cuda.current_stream(x.device).cuda_stream)
+    if rc:
+        _native.check(rc, "hy_linear_add")
+    return y

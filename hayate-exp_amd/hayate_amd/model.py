@@ -20,7 +20,8 @@ from dataclasses import dataclass
 import torch
 import torch.nn as nn
 
-from .attention import GroupedQueryAttention
+from . import linear
+from .attention import GroupedQueryAttention, _norm_eps
 from .rope import compute_rope_params
 
 
@@ -67,6 +68,8 @@ class TransformerBlock(nn.Module):
 
     def forward(self, x, cos, sin, position_ids, prev_k, prev_v, varlen_metadata=None,
                 paged_cache=None, layer_idx=None):
+        if paged_cache is not None and linear.few_rows(x) and self._few_rows_fit(x):
+            return self._few_rows(x, cos, sin, paged_cache, layer_idx), None, None
         shortcut = x
         x, new_k, new_v = self.self_attn(self.input_layernorm(x), cos, sin, position_ids, prev_k,
                                          prev_v, varlen_metadata, paged_cache, layer_idx)
@@ -74,6 +77,45 @@ class TransformerBlock(nn.Module):
         shortcut = x
         x = self.mlp(self.post_attention_layernorm(x)) + shortcut
         return x, new_k, new_v
+
+    def _few_rows_fit(self, x) -> bool:
+        """Whether the fused path below computes what the modules would."""
+        attn, mlp = self.self_attn, self.mlp
+        if type(attn) is not GroupedQueryAttention or type(mlp) is not FeedForward or x.dim() != 3:
+            return False
+        qkv = (attn.q_proj, attn.k_proj, attn.v_proj)
+        if not linear.plain(x, modules=(attn, mlp),
+                            norms=(self.input_layernorm, self.post_attention_layernorm),
+                            linears=(*qkv, attn.o_proj, mlp.gate_proj, mlp.up_proj,
+                                     mlp.down_proj)):
+            return False
+        rows, d = x.shape[0] * x.shape[1], x.shape[2]
+        heads, mid = attn.num_heads * attn.head_dim, mlp.gate_proj.weight.shape[0]
+        return (linear.norm_fits(d, rows) and linear.add_fits(heads, rows)
+                and linear.add_fits(mid, rows)
+                and all(lin.weight.shape[1] == d for lin in qkv)
+                and attn.q_proj.weight.shape[0] == heads
+                and attn.o_proj.weight.shape == (d, heads)
+                and mlp.gate_proj.weight.shape == mlp.up_proj.weight.shape == (mid, d)
+                and mlp.gate_proj.weight.stride() == mlp.up_proj.weight.stride()
+                and mlp.down_proj.weight.shape == (d, mid))
+
+    def _few_rows(self, x, cos, sin, paged_cache, layer_idx):
+        """The block for a decode tick's few rows: norms, silu and residuals
+        inside the four products, two launches beside the attention's own per
+        half of the block."""
+        attn, mlp, shape = self.self_attn, self.mlp, x.shape
+        norm = self.input_layernorm
+        x = linear.rows_of(x)
+        qkv = linear.norm_linear(x, norm.weight, _norm_eps(norm, x.dtype),
+                                 attn.fused_qkv_weight())
+        context = attn.context(*attn.split_qkv(qkv.view(*shape[:2], -1)), cos, sin, paged_cache,
+                               layer_idx)
+        x = linear.linear_add(linear.rows_of(context), attn.o_proj.weight, x)
+        norm = self.post_attention_layernorm
+        h = linear.norm_linear(x, norm.weight, _norm_eps(norm, x.dtype), mlp.gate_proj.weight,
+                               mlp.up_proj.weight)
+        return linear.linear_add(h, mlp.down_proj.weight, x).view(shape)
 
 
 class Qwen3Model(nn.Module):
@@ -120,6 +162,12 @@ class Qwen3Model(nn.Module):
             x = x[0].index_select(0, last).unsqueeze(1)
         else:
             x = x[:, -1:, :]
+        if (linear.few_rows(x) and linear.plain(x, norms=(self.norm,), linears=(self.out_head,))
+                and linear.norm_fits(x.shape[-1], x.shape[0])
+                and self.out_head.weight.shape[1] == x.shape[-1]):
+            logits = linear.norm_linear(linear.rows_of(x), self.norm.weight,
+                                        _norm_eps(self.norm, x.dtype), self.out_head.weight)
+            return logits.unsqueeze(1), None, None
         return self.out_head(self.norm(x)), None, None
 
 

@@ -339,6 +339,36 @@ int hy_paged_prefill_merge(void *out, int64_t o_stride_seq, int64_t o_stride_tok
                            int32_t num_kv_heads, int32_t head_dim,
                            void *stream);
 
+/*
+ * Products of few rows (the tokens of a decode tick) with the weights around
+ * attention. x is m rows of k bf16 values x_stride apart, weights are rows of
+ * k values w_stride apart (torch's Linear layout); both 16-byte aligned with
+ * strides that are multiples of 8. fp32 sums, one rounding of the result.
+ *
+ * hy_norm_linear: y[m][n] = norm(x) W^T with norm the RMSNorm of each row by
+ * norm_weight (k values) and eps, or x itself when norm_weight is NULL; with
+ * up_weight (same shape and stride as weight) y = silu(norm(x) W^T) *
+ * (norm(x) up_weight^T). k is a multiple of 64 in 512 .. 4096 and m at most 32
+ * (16 when k > 3072); other sizes return HY_EUNSUPPORTED.
+ * Replaces input_layernorm + the q/k/v projections, post_attention_layernorm
+ * + gate_proj, up_proj and silu (hayate/model/block.py:33-58, attention.py:58-60,
+ * linear.py:18-22) and norm + out_head (qwen.py:162-165) for such ticks.
+ */
+int hy_norm_linear(const void *x, int64_t x_stride, int32_t m, int32_t k,
+                   const void *norm_weight, float eps, const void *weight,
+                   const void *up_weight, int64_t w_stride, int32_t n, void *y,
+                   int64_t y_stride, void *stream);
+
+/*
+ * y[m][n] = x W^T + residual (residual may be NULL): k a multiple of 128, m at
+ * most 32; other sizes return HY_EUNSUPPORTED. Replaces o_proj and
+ * down_proj with the residual additions of block.py:45-58.
+ */
+int hy_linear_add(const void *x, int64_t x_stride, int32_t m, int32_t k,
+                  const void *weight, int64_t w_stride, int32_t n,
+                  const void *residual, int64_t r_stride, void *y,
+                  int64_t y_stride, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
