@@ -34,18 +34,23 @@
 // wait and one barrier per tile. The fourth stage keeps a tile's V rows in
 // place while the next tile's first block runs their P V (below). A load
 // instruction writes 64 lanes x 16 bytes to consecutive LDS addresses, so
-// the bank-conflict-free layouts are
-// lane permutations instead of padded rows (16-byte units, "chunk" = 8
-// dims):
-//   K: unit(row, chunk) = (row / 16) * 256 + chunk * 16 + row % 16. The
-//      K-operand read (16 lanes = 16 rows, one chunk) touches 16
-//      consecutive units; one load instruction = 16 rows x 4 chunks
-//      (64-byte runs of each row).
-//   V: unit(row, chunk) = (row / 4) * 64 + chunk * 4 + row % 4. The
-//      transposing read (32 lanes = 4 rows x 32 dims) touches 16
-//      consecutive units; one load instruction = 4 whole rows.
-// Both give per-lane base addresses with compile-time offsets for every
-// block, dim slice and row group. The block loop is software-pipelined: a
+// the bank-conflict-free layouts are lane permutations instead of padded rows.
+// Four neighbouring lanes must stay within 64 bytes of one row: with lanes
+// going down the rows instead, a load takes a CU three times as long (34
+// against 105 GB/s from L2). With it Q (through LDS instead of eight strided
+// register loads) and the tiles cost a workgroup 2 us less before its first
+// block: a 512-token chunk 26.0 -> 24.0 us, a 2-token one 11.6 -> 9.6 us,
+// 4 x 512 at offsets 0-3584 95.0 -> 93.3 us, 8 x 512 205 -> 202 us (graph steps,
+// append and merges included). In 16-byte units, "chunk" = 8 dims:
+//   K: unit(row, chunk) = (row / 16) * 256 + (chunk / 4) * 64 + (row % 16) * 4
+//      + (chunk % 4 ^ row / 4 % 4). One load instruction = 16 rows x 4 chunks;
+//      the K-operand read (16 lanes = 16 rows, one chunk) touches every bank
+//      once. Q, loaded the same way before the first tiles, likewise.
+//   V: unit(row, chunk) = (row / 4) * 64 + (chunk / 4) * 16 + (row % 4) * 4 +
+//      chunk % 4. One load instruction = 4 whole rows; the transposing read
+//      (32 lanes = 4 rows x 32 dims) touches 16 consecutive units.
+// Per-lane base addresses (two for K, one for V) with compile-time offsets
+// reach every block, dim slice and row group. The block loop is software-pipelined: a
 // wave computes block j + 1's scores on the matrix core while its VALU
 // turns block j's scores into probabilities (see the block body below).
 // The softmax rescales lazily: the exponent base of a row only moves when
@@ -198,28 +203,11 @@ void prefill_kernel(
   const int c = lane & 31;
   const int h = lane >> 5;
 
-  // This lane's row and its Q^T operand (zeros for rows past the chunk).
+  // This lane's row.
   const int r = 32 * wave + c;
   const int row_tok = q_begin + r / G;
   const bool live = row_tok < q_end;
-  bf16x8 qop[8];
-  {
-    // rows past the chunk read the chunk's first row (in bounds) and are
-    // zeroed, so the eight loads issue together without a branch
-    const uint16_t *src = q + seq * q_ss +
-                          static_cast<int64_t>(qs + (live ? row_tok : q_begin)) * q_st +
-                          (h0 + r % G) * q_sh;
-    u32x4 raw[8];
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) raw[kk] = load16(src + 16 * kk + 8 * h);
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      u32x4 w = raw[kk];
-      if (!live) w = u32x4{0u, 0u, 0u, 0u};
-      qop[kk] = __builtin_bit_cast(bf16x8, w);
-    }
-  }
-
+  bf16x8 qop[8];  // this lane's row of Q^T (zeros for rows past the chunk)
   f32x16 acc[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db)
@@ -257,9 +245,9 @@ void prefill_kernel(
   const int page_mask = (1 << page_shift) - 1;
   const int n_tiles = (kv_end - kv_begin + kTile - 1) / kTile;
 
-  // Tile loads: wave w issues K instructions 2w, 2w + 1 (rows 16 (w / 2) +
-  // lane % 16, chunks 4 (i % 4) + lane / 16) and V instructions 2w, 2w + 1
-  // (rows 4 i + lane % 4, chunk lane / 4). A wave's rows lie in one page
+  // Tile loads: wave w issues K instructions 2w, 2w + 1 (instruction i: rows 16
+  // (i / 4) + lane / 4, chunks of 4 (i % 4) ..) and V instructions 2w, 2w + 1
+  // (rows 4 i + lane / 4 % 4, every chunk). A wave's rows lie in one page
   // (pages hold >= 32 keys), so each tensor needs one page id per tile;
   // they are fetched a tile ahead. Rows at or past kv_end load the last
   // valid key (any finite data: their scores are masked).
@@ -276,36 +264,41 @@ void prefill_kernel(
     pg.v = static_cast<uint32_t>(pt[max(min(kt + 8 * wave, last_key), 0) >> page_shift]);
     return pg;
   };
+  // First element of this lane's chunk within its row.
+  const int k_chunk = 8 * ((lane & 3) ^ ((lane >> 4) & 3));
+  const int v_chunk = 32 * (lane >> 4) + 8 * (lane & 3);
   auto issue_tile = [&](int kt, const Pages &pg, uint16_t *dst) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int i = 2 * wave + j;
       {
-        const int key = min(kt + 16 * (i >> 2) + (lane & 15), last_key);
+        const int key = min(kt + 16 * (i >> 2) + (lane >> 2), last_key);
         const int64_t p = (static_cast<int64_t>(pg.k) << page_shift) + (key & page_mask);
-        load_to_lds(kh + p * kHeadDim + 8 * (4 * (i & 3) + (lane >> 4)), dst + i * 512);
+        load_to_lds(kh + p * kHeadDim + 32 * (i & 3) + k_chunk, dst + i * 512);
       }
       {
-        const int key = min(kt + 4 * i + (lane & 3), last_key);
+        const int key = min(kt + 4 * i + ((lane >> 2) & 3), last_key);
         const int64_t p = (static_cast<int64_t>(pg.v) << page_shift) + (key & page_mask);
-        load_to_lds(vh + p * kHeadDim + 8 * (lane >> 2), dst + kTile * kHeadDim + i * 512);
+        load_to_lds(vh + p * kHeadDim + v_chunk, dst + kTile * kHeadDim + i * 512);
       }
     }
   };
 
-  // Per-lane LDS read bases (u16 units). K operand of row c, dims 16 kk +
-  // 8 h: unit (c / 16) * 256 + (2 kk + h) * 16 + c % 16, i.e. base + 256 kk.
-  // V^T transposed read of lane (q16, r16): row 4 (q16 / 2) + r16 / 4 (+ 8
-  // for the second half, + 16 kh2, + 32 kb), dims 16 (q16 % 2) + 4 (r16 % 4)
-  // (+ 32 db), i.e. base + 1024 hi + 2048 kh2 + 128 db.
+  // Per-lane LDS read bases (u16 units). K operand of row c, chunk 2 kk + h:
+  // k_base[kk % 2] + 512 (kk / 2). V^T transposed read of lane (q16, r16): row
+  // 4 (q16 / 2) + r16 / 4 (+ 8 for the second half, + 16 kh2, + 32 kb), dims
+  // 32 db + 16 (q16 % 2) + 4 (r16 % 4): v_base + 1024 hi + 2048 kh2 + 128 db.
   const int r16 = lane & 15;
   const int q16 = lane >> 4;
-  const int k_base = (c >> 4) * 2048 + h * 128 + (c & 15) * 8;
-  const int v_base = 512 * (q16 >> 1) + 64 * (q16 & 1) + 32 * ((r16 & 3) >> 1) + 8 * (r16 >> 2) +
+  int k_base[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    k_base[i] = (c >> 4) * 2048 + (c & 15) * 32 + 8 * ((2 * i + h) ^ ((c >> 2) & 3));
+  const int v_base = 512 * (q16 >> 1) + 32 * (r16 >> 2) + 16 * (q16 & 1) + 8 * ((r16 & 3) >> 1) +
                      4 * (r16 & 1);
   // Block j's K and V rows in the ring: stage (j / 2) % kStages, half j % 2.
   auto k_block = [&](int j) -> const uint16_t * {
-    return smem + ((j >> 1) % kStages) * kStage + 4096 * (j & 1) + k_base;
+    return smem + ((j >> 1) % kStages) * kStage + 4096 * (j & 1);
   };
   auto v_block = [&](int j) -> const uint16_t * {
     return smem + ((j >> 1) % kStages) * kStage + kTile * kHeadDim + 4096 * (j & 1) + v_base;
@@ -326,7 +319,8 @@ void prefill_kernel(
   auto read_k = [&](int j) __attribute__((always_inline)) {
     const uint16_t *kb = k_block(j);
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) kop[kk] = *reinterpret_cast<const bf16x8 *>(kb + 256 * kk);
+    for (int kk = 0; kk < 8; ++kk)
+      kop[kk] = *reinterpret_cast<const bf16x8 *>(kb + k_base[kk & 1] + 512 * (kk >> 1));
   };
   auto qk = [&]() __attribute__((always_inline)) {
     f32x16 s;
@@ -477,9 +471,27 @@ void prefill_kernel(
   const Pages pg0 = fetch_pages(kv_begin);
   const Pages pg1 = fetch_pages(kv_begin + kTile);
   Pages pg_next = fetch_pages(kv_begin + 2 * kTile);
+  // This wave's 32 Q rows go through the last two stages (no tile uses them
+  // before the first barrier), laid out as a K block. Rows past the chunk
+  // read its first token (in bounds) and are zeroed.
+  uint16_t *q_lds = smem + 2 * kStage + 32 * kHeadDim * wave;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int row = 32 * wave + 16 * (i >> 2) + (lane >> 2);
+    const int tok = q_begin + row / G;
+    load_to_lds(q + seq * q_ss + static_cast<int64_t>(qs + (tok < q_end ? tok : q_begin)) * q_st +
+                    (h0 + row % G) * q_sh + 32 * (i & 3) + k_chunk,
+                q_lds + i * 512);
+  }
   if (n_tiles > 0) issue_tile(kv_begin, pg0, smem);
   if (n_tiles > 1) issue_tile(kv_begin + kTile, pg1, smem + kStage);
   wait_tile_loads();
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) {
+    u32x4 w = *reinterpret_cast<const u32x4 *>(q_lds + k_base[kk & 1] + 512 * (kk >> 1));
+    if (!live) w = u32x4{0u, 0u, 0u, 0u};
+    qop[kk] = __builtin_bit_cast(bf16x8, w);
+  }
   __syncthreads();
   read_k(0);
   s_a = qk();
