@@ -176,7 +176,7 @@ void prefill_kernel(
     const uint16_t *__restrict__ k_pool, const uint16_t *__restrict__ v_pool,
     int64_t pool_hs, const int32_t *__restrict__ page_table, int64_t pt_stride,
     const int32_t *__restrict__ items, float *__restrict__ ws_acc, float *__restrict__ ws_ml,
-    int num_kv_heads, int page_shift, float scale_log2) {
+    int num_kv_heads, int page_shift, float scale_log2, bool q_aligned) {
   static_assert(kThreads == 512, "eight waves");
   __shared__ __attribute__((aligned(1024))) uint16_t smem[kStages * kStage];
 
@@ -479,9 +479,13 @@ void prefill_kernel(
   for (int i = 0; i < 8; ++i) {
     const int row = 32 * wave + 16 * (i >> 2) + (lane >> 2);
     const int tok = q_begin + row / G;
-    load_to_lds(q + seq * q_ss + static_cast<int64_t>(qs + (tok < q_end ? tok : q_begin)) * q_st +
-                    (h0 + row % G) * q_sh + 32 * (i & 3) + k_chunk,
-                q_lds + i * 512);
+    const uint16_t *src = q + seq * q_ss +
+                          static_cast<int64_t>(qs + (tok < q_end ? tok : q_begin)) * q_st +
+                          (h0 + row % G) * q_sh + 32 * (i & 3) + k_chunk;
+    if (q_aligned)
+      load_to_lds(src, q_lds + i * 512);
+    else  // rows off 16 bytes: through registers
+      *reinterpret_cast<u32x4 *>(q_lds + i * 512 + 8 * lane) = load16(src);
   }
   if (n_tiles > 0) issue_tile(kv_begin, pg0, smem);
   if (n_tiles > 1) issue_tile(kv_begin + kTile, pg1, smem + kStage);
@@ -531,42 +535,59 @@ void prefill_kernel(
   // Epilogue: full row sums, then the output or the split's partial.
   const float lsum = halves_sum(l_run);
   if (slot < 0) {
-    if (!live) return;
+    // The output rows go through LDS so that 16 lanes store a row: a lane
+    // holds 8-byte pieces of one row, and 64 lanes storing to 32 rows keep a
+    // CU's memory pipe busy four times as long. The two stages after the last
+    // tile's are free (their tiles were left before the last barrier); 8 KiB
+    // a wave, 16-byte units with unit(row, chunk) = row * 16 + (chunk ^ row % 16).
+    // With the partials below: a 512-token chunk 24.0 -> 21.9 us, 20 of them
+    // 137 -> 125 us, 4 x 512 at offsets 0-3584 94.3 -> 93.0 us (graph steps).
     const float inv = 1.0f / lsum;
-    uint16_t *dst = out + seq * o_ss + static_cast<int64_t>(qs + row_tok) * o_st +
-                    (h0 + r % G) * o_sh;
+    uint16_t *o_lds = smem + ((n_tiles + (wave >> 2)) % kStages) * kStage +
+                      32 * kHeadDim * (wave & 3);
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int j = 0; j < 16; ++j) {
+      const int db = j >> 2, i = 4 * (j & 3);
+      const uint32_t w0 = pack_bf16x2_rne(acc[db][i] * inv, acc[db][i + 1] * inv);
+      const uint32_t w1 = pack_bf16x2_rne(acc[db][i + 2] * inv, acc[db][i + 3] * inv);
+      *reinterpret_cast<uint2 *>(o_lds + c * kHeadDim + 8 * (j ^ (c & 15)) + 4 * h) =
+          make_uint2(w0, w1);
+    }
 #pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int d = 32 * db + 8 * i4 + 4 * h;
-        const uint32_t w0 = pack_bf16x2_rne(acc[db][4 * i4] * inv, acc[db][4 * i4 + 1] * inv);
-        const uint32_t w1 =
-            pack_bf16x2_rne(acc[db][4 * i4 + 2] * inv, acc[db][4 * i4 + 3] * inv);
-        *reinterpret_cast<uint2 *>(dst + d) = make_uint2(w0, w1);
-      }
+    for (int i = 0; i < 8; ++i) {
+      const int row = 4 * i + (lane >> 4);
+      const int chunk = lane & 15;
+      const int tok = q_begin + (32 * wave + row) / G;
+      const u32x4 w =
+          *reinterpret_cast<const u32x4 *>(o_lds + row * kHeadDim + 8 * (chunk ^ (row & 15)));
+      if (tok < q_end)
+        store16(out + seq * o_ss + static_cast<int64_t>(qs + tok) * o_st +
+                    (h0 + (32 * wave + row) % G) * o_sh + 8 * chunk,
+                w);
+    }
   } else {
-    const int64_t pr = (static_cast<int64_t>(slot) * num_kv_heads + kvh) * kRows + r;
-    float *dst = ws_acc + pr * kHeadDim;
+    // Partials keep the accumulator's own order: per wave, 16 groups of four
+    // dims (32 db + 8 i4 + 4 h ..), each 64 lanes x 16 bytes.
+    const int64_t pr = (static_cast<int64_t>(slot) * num_kv_heads + kvh) * kRows;
+    float *dst = ws_acc + (pr + 32 * wave) * kHeadDim + 4 * lane;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) {
-        const int d = 32 * db + 8 * i4 + 4 * h;
-        *reinterpret_cast<f32x4 *>(dst + d) =
-            f32x4{acc[db][4 * i4], acc[db][4 * i4 + 1], acc[db][4 * i4 + 2],
-                  acc[db][4 * i4 + 3]};
-      }
+    for (int j = 0; j < 16; ++j) {
+      const int db = j >> 2, i = 4 * (j & 3);
+      *reinterpret_cast<f32x4 *>(dst + 256 * j) =
+          f32x4{acc[db][i], acc[db][i + 1], acc[db][i + 2], acc[db][i + 3]};
+    }
     if (h == 0) {
-      ws_ml[pr * 2 + 0] = base;
-      ws_ml[pr * 2 + 1] = lsum;
+      ws_ml[(pr + r) * 2 + 0] = base;
+      ws_ml[(pr + r) * 2 + 1] = lsum;
     }
   }
 }
 
 // Combines the splits of a query tile: grid (kv head, merge item, kRows /
-// 32 row groups), 512 threads = 32 rows x 16 lanes x 8 dims. Item = {seq,
-// q_begin, q_end, first_slot, num_splits, q_row = q_start[seq], 0, 0}.
+// 32 row groups), 512 threads = 16 groups of 8 dims x 32 rows, in the order
+// the prefill waves left their partials; the merged rows go through LDS so
+// that 16 lanes store one. Item = {seq, q_begin, q_end, first_slot,
+// num_splits, q_row = q_start[seq], 0, 0}.
 // Splits are loaded kMergeRound at a time in rounds of independent loads:
 // every load reads a real split (the index is clamped to the last one; a
 // partial holds all kRows rows, so rows past q_end are in bounds too) and
@@ -591,9 +612,9 @@ __global__ __launch_bounds__(512) void prefill_merge_kernel(
   const int nsplit = it1.x;
   // an empty record pads a list to a fixed launch size
   if (q_end <= q_begin || nsplit <= 0) return;
-  const int r = 32 * blockIdx.z + (threadIdx.x >> 4);
-  const int d = (threadIdx.x & 15) * 8;
-  const int i = q_begin + r / G;
+  __shared__ __attribute__((aligned(16))) uint16_t rows[32 * kHeadDim];
+  const int c = threadIdx.x & 31;  // row of the group
+  const int j8 = threadIdx.x >> 5;  // dims 8 j8 ..
   const int64_t qs = it1.y;  // q_start[seq], carried by the item
   float mx = -INFINITY, lsum = 0.f;
   f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
@@ -603,12 +624,14 @@ __global__ __launch_bounds__(512) void prefill_merge_kernel(
 #pragma unroll
     for (int j = 0; j < kMergeRound; ++j) {
       const int64_t pr =
-          (static_cast<int64_t>(first + min(s0 + j, nsplit - 1)) * num_kv_heads + kvh) * kRows + r;
-      const float2 ml = *reinterpret_cast<const float2 *>(ws_ml + pr * 2);
+          (static_cast<int64_t>(first + min(s0 + j, nsplit - 1)) * num_kv_heads + kvh) * kRows +
+          32 * blockIdx.z;
+      const float2 ml = *reinterpret_cast<const float2 *>(ws_ml + (pr + c) * 2);
       m[j] = ml.x;
       l[j] = ml.y;
-      x0[j] = *reinterpret_cast<const f32x4 *>(ws_acc + pr * kHeadDim + d);
-      x1[j] = *reinterpret_cast<const f32x4 *>(ws_acc + pr * kHeadDim + d + 4);
+      const float *src = ws_acc + pr * kHeadDim + 256 * j8 + 4 * c;
+      x0[j] = *reinterpret_cast<const f32x4 *>(src);
+      x1[j] = *reinterpret_cast<const f32x4 *>(src + 128);
     }
 #pragma unroll
     for (int j = 0; j < kMergeRound; ++j) {
@@ -635,11 +658,17 @@ __global__ __launch_bounds__(512) void prefill_merge_kernel(
     }
     mx = cmx;
   }
-  if (i >= q_end) return;
-  uint16_t *dst = out + seq * o_ss + (qs + i) * o_st + (kvh * G + r % G) * o_sh + d;
-  *reinterpret_cast<u32x4 *>(dst) =
+  *reinterpret_cast<u32x4 *>(rows + c * kHeadDim + 8 * (j8 ^ (c & 15))) =
       u32x4{pack_bf16x2_rne(a0[0] / lsum, a0[1] / lsum), pack_bf16x2_rne(a0[2] / lsum, a0[3] / lsum),
             pack_bf16x2_rne(a1[0] / lsum, a1[1] / lsum), pack_bf16x2_rne(a1[2] / lsum, a1[3] / lsum)};
+  __syncthreads();
+  const int r = threadIdx.x >> 4;
+  const int chunk = threadIdx.x & 15;
+  const int row = 32 * blockIdx.z + r;
+  const int i = q_begin + row / G;
+  if (i >= q_end) return;
+  store16(out + seq * o_ss + (qs + i) * o_st + (kvh * G + row % G) * o_sh + 8 * chunk,
+          *reinterpret_cast<const u32x4 *>(rows + r * kHeadDim + 8 * (chunk ^ (r & 15))));
 }
 
 template <int G>
@@ -649,10 +678,13 @@ void launch_prefill(hipStream_t st, int num_kv_heads, int n_items, const uint16_
                     int64_t pool_hs, const int32_t *page_table, int64_t pt_stride,
                     const int32_t *items, float *ws_acc, float *ws_ml, int page_shift,
                     float scale_log2) {
+  const bool q_aligned =
+      (reinterpret_cast<uintptr_t>(q) & 15) == 0 && ((q_ss | q_st | q_sh) & 7) == 0;
   hipLaunchKernelGGL((prefill_kernel<G>), dim3(num_kv_heads, n_items), dim3(kThreads), 0,
                      st, q, q_ss,
                      q_st, q_sh, out, o_ss, o_st, o_sh, k_pool, v_pool, pool_hs, page_table,
-                     pt_stride, items, ws_acc, ws_ml, num_kv_heads, page_shift, scale_log2);
+                     pt_stride, items, ws_acc, ws_ml, num_kv_heads, page_shift, scale_log2,
+                     q_aligned);
 }
 
 template <int G>
