@@ -22,20 +22,24 @@ from . import _native
 MAX_ROWS = 32
 
 
-def few_rows(x: torch.Tensor) -> bool:
-    """True when `x` (..., d) is a plain bf16 tensor of at most MAX_ROWS rows on
-    the current HIP device and nothing watches the operators run on it
-    (gradients, autocast, tracing, dispatch or function modes, functorch)."""
-    if (type(x) is not torch.Tensor or x.dtype is not torch.bfloat16 or not x.is_cuda
-            or not 0 < x.numel() <= MAX_ROWS * x.shape[-1]
-            or torch.is_grad_enabled() or torch.is_autocast_enabled()):
-        return False
+def unwatched() -> bool:
+    """True when nothing watches the operators a call runs: tracing, dispatch or
+    function modes, functorch, forward-mode gradients."""
     c = torch._C
     return (c._len_torch_dispatch_stack() == 0 and c._len_torch_function_stack() == 0
             and c._get_tracing_state() is None and not torch.compiler.is_compiling()
             and torch.autograd.forward_ad._current_level < 0
-            and c._functorch.peek_interpreter_stack() is None
-            and x.device.index == torch.cuda.current_device())
+            and c._functorch.peek_interpreter_stack() is None)
+
+
+def few_rows(x: torch.Tensor) -> bool:
+    """True when `x` (..., d) is a plain bf16 tensor of at most MAX_ROWS rows on
+    the current HIP device and nothing watches the operators run on it, nor
+    gradients or autocast change them."""
+    return (type(x) is torch.Tensor and x.dtype is torch.bfloat16 and x.is_cuda
+            and 0 < x.numel() <= MAX_ROWS * x.shape[-1]
+            and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
+            and unwatched() and x.device.index == torch.cuda.current_device())
 
 
 def _bare(m: nn.Module) -> bool:

@@ -12,7 +12,9 @@ Semantics of the reference's hayate/engine/sampler.py:
 The reference loops over rows in Python, one small kernel chain per row
 (:67-85). Here every row of the batch goes through one sort and a handful of
 batched ops, with per-row temperature / k / p as tensors, so a tick costs
-the same few launches whatever the batch size.
+the same few launches whatever the batch size. 16-bit logits on a HIP device
+(the engine's) take hy_sample instead: one launch, no sort, the same draws
+from the same generator.
 """
 
 from __future__ import annotations
@@ -20,7 +22,10 @@ from __future__ import annotations
 import math
 from typing import Optional, Sequence
 
+import numpy as np
 import torch
+
+from . import _native, linear
 
 
 def validate_parameters(temperature, top_k, top_p) -> None:
@@ -47,6 +52,8 @@ def sample_batch(logits: torch.Tensor, temperature: Sequence[float],
                  top_k: Sequence[Optional[int]], top_p: Sequence[Optional[float]],
                  generator: Optional[torch.Generator] = None) -> torch.Tensor:
     """One token id per row of logits (n, vocab) -> int64 (n, 1)."""
+    if _native_rows(logits, temperature, top_k, top_p):
+        return _sample_native(logits, temperature, top_k, top_p, generator)
     n, vocab = logits.shape
     dev = logits.device
     greedy_rows = [i for i, t in enumerate(temperature) if t == 0]
@@ -76,6 +83,52 @@ def sample_batch(logits: torch.Tensor, temperature: Sequence[float],
     scores = scores.masked_fill(~keep | remove, -torch.inf)
     drawn = torch.multinomial(torch.softmax(scores, dim=-1), 1, generator=generator)
     out.index_copy_(0, idx, drawn)
+    return out
+
+
+_DTYPES = {torch.bfloat16: 0, torch.float16: 1}
+MAX_VOCAB = 4_194_304
+
+
+def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
+    """True when hy_sample takes these rows: 16-bit logits on the current HIP
+    device, contiguous along the vocabulary, temperatures whose scores keep
+    the logits' order (outside [1e-30, 1e30] they vanish or overflow and become
+    equal), and nothing watching the ops."""
+    return (type(logits) is torch.Tensor and logits.dtype in _DTYPES and logits.is_cuda
+            and logits.dim() == 2 and logits.shape[0] > 0 and 0 < logits.shape[1] <= MAX_VOCAB
+            and logits.stride(1) == 1
+            and len(temperature) == len(top_k) == len(top_p) == logits.shape[0]
+            and all(t == 0 or 1e-30 <= t <= 1e30 for t in temperature)
+            and all(k is None or k >= 1 for k in top_k)
+            and all(p is None or p > 0 for p in top_p)
+            and linear.unwatched() and logits.device.index == torch.cuda.current_device())
+
+
+def _sample_native(logits, temperature, top_k, top_p, generator):
+    n, vocab = logits.shape
+    dev = logits.device
+    temp = np.asarray(temperature, dtype=np.float32)
+    k = np.asarray([vocab if v is None else min(v, vocab) for v in top_k], dtype=np.int32)
+    p = np.asarray([1.0 if v is None else v for v in top_p], dtype=np.float32)
+    drawn = int(np.count_nonzero(temp))
+    noise = valid = None
+    if drawn:
+        # the noise torch.multinomial draws for these rows' probabilities
+        noise = torch.empty((drawn, vocab), device=dev).exponential_(1, generator=generator)
+        valid = torch.empty((), dtype=torch.bool, device=dev)
+    out = torch.empty((n, 1), dtype=torch.long, device=dev)
+    lib = _native.lib()
+    work = torch.empty(lib.hy_sample_workspace_bytes(n, vocab), dtype=torch.uint8, device=dev)
+    rc = lib.hy_sample(
+        logits.data_ptr(), logits.stride(0), _DTYPES[logits.dtype], n, vocab, temp.ctypes.data,
+        k.ctypes.data, p.ctypes.data, noise.data_ptr() if drawn else None, out.data_ptr(),
+        valid.data_ptr() if drawn else None, work.data_ptr(), work.numel(),
+        torch.cuda.current_stream(dev).cuda_stream)
+    if rc:
+        _native.check(rc, "hy_sample")
+    if drawn:
+        torch._assert_async(valid, "logits hold NaN or have no finite maximum")
     return out
 
 

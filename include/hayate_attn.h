@@ -369,6 +369,31 @@ int hy_linear_add(const void *x, int64_t x_stride, int32_t m, int32_t k,
                   const void *residual, int64_t r_stride, void *y,
                   int64_t y_stride, void *stream);
 
+/*
+ * One token per row of 16-bit logits (dtype 0: bf16, 1: fp16; rows row_stride
+ * apart, values contiguous). temperature, top_k and top_p are host arrays of
+ * n_rows entries, read before the call returns. temperature 0: the first
+ * largest logit (a NaN counts as the largest). Otherwise scores are logits /
+ * temperature; top-k keeps every score >= the k-th largest (top_k >= vocab: all);
+ * top-p the shortest prefix of the descending order (equal scores by index) whose
+ * mass exceeds top_p (>= 1: all); the token is the largest p / noise over the
+ * kept ones, p their softmax. noise holds exponential(1) variates, `vocab` for
+ * each row with a temperature, in row order (so the draw is the one that
+ * torch.multinomial makes of that noise). *valid becomes 1, or 0 if a row with a
+ * temperature has a NaN or no finite maximum; its token is then meaningless.
+ * noise and valid may be NULL when every row is greedy. workspace is device
+ * memory of hy_sample_workspace_bytes(n_rows, vocab), 8-byte aligned.
+ * Temperatures outside [1e-30, 1e30] and vocabularies past 4,194,304 return
+ * HY_EUNSUPPORTED.
+ * Replaces Sampler.sample (hayate/engine/sampler.py:39-85).
+ */
+int hy_sample(const void *logits, int64_t row_stride, int32_t dtype,
+              int32_t n_rows, int32_t vocab, const float *temperature,
+              const int32_t *top_k, const float *top_p, const float *noise,
+              int64_t *out, uint8_t *valid, void *workspace,
+              int64_t workspace_bytes, void *stream);
+int64_t hy_sample_workspace_bytes(int32_t n_rows, int32_t vocab);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,135 @@
+"""hy_sample (csrc/sample.hip) against the sort-based path of sample_batch, which
+32-bit copies of the same logits take, on the same generator state: the same
+draws, since the noise and the order of p / q are the same.
+
+Where a top-p cut falls within rounding of a token's mass the two may keep one
+token more or less (sums of up to 151,936 fp32 terms in another order: below
+1e-5 of the mass), and small vocabularies are sorted by an unstable sort, which
+splits equal scores at the cut differently. So a differing row is accepted
+if both tokens are kept by a float64 cut with that slack.
+"""
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from hayate_amd import _native
+    from hayate_amd.sampler import sample_batch
+
+DEV = "cuda"
+SETTINGS = [(0.0, None, None), (1.0, None, None), (0.7, 1, None), (0.7, 20, None),
+            (1.3, 50, 0.8), (1.0, None, 0.05), (0.6, None, 0.5), (1.0, None, 0.95),
+            (2.0, 10_000_000, 0.999), (0.3, None, 1.0), (1.0, "half", 0.9), (5.0, "all", None)]
+
+
+def settings(vocab):
+    fix = {"half": vocab // 2 + 1, "all": vocab}
+    return [(t, fix.get(k, k), p) for t, k, p in SETTINGS]
+
+
+def kept(row, t, k, p, token, slack=1e-5):
+    x = row.double()
+    s = x / t
+    if k is not None and k < x.numel() and x[token] < torch.topk(x, k).values[-1]:
+        return False
+    if k is not None and k < x.numel():
+        s = s.masked_fill(x < torch.topk(x, k).values[-1], -math.inf)
+    mass = torch.softmax(s, 0)
+    above = float(mass[x > x[token]].sum())
+    return p is None or p >= 1 or above <= p + slack
+
+
+def check(logits, seed):
+    rows = settings(logits.shape[1])
+    t, k, p = map(list, zip(*(rows * (logits.shape[0] // len(rows) + 1))[: logits.shape[0]]))
+    gens = [torch.Generator(device=DEV).manual_seed(seed) for _ in range(2)]
+    a = sample_batch(logits, t, k, p, gens[0])
+    b = sample_batch(logits.float(), t, k, p, gens[1])
+    assert a.shape == b.shape and a.dtype == b.dtype
+    # both consumed the same noise
+    assert torch.equal(gens[0].get_state(), gens[1].get_state())
+    differ = (a != b).flatten().nonzero().flatten().tolist()
+    for r in differ:
+        assert t[r] != 0 and p[r] is not None and p[r] < 1
+        for token in (int(a[r]), int(b[r])):
+            assert kept(logits[r], t[r], k[r], p[r], token), (r, t[r], k[r], p[r], token)
+    return len(differ)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("vocab", [1, 2, 9, 1000, 8191, 8193, 32_771, 151_936])
+def test_draws_equal_the_sorted_path(vocab, dtype):
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    n = 3 * len(SETTINGS)
+    wide = (torch.randn(n, vocab + 3, generator=g, device=DEV) * 2.5).to(getattr(torch, dtype))
+    logits = wide[:, 1 : vocab + 1]  # rows at any alignment
+    differ = sum(check(logits, s) for s in range(3))
+    if vocab >= 1000:  # no row of these sits at a rounding decision
+        assert differ <= 1
+
+
+@pytest.mark.parametrize("value", [0.0, -0.0, 3.0, -2.0])
+def test_counters_that_overflow(value):
+    """More than 65,535 logits of one value: counted again in 32 bits."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x = torch.full((2 * len(SETTINGS), 151_936), value, device=DEV)
+    x[:, ::4] = torch.randn(x.shape[0], x.shape[1] // 4, generator=g, device=DEV)
+    if value == 0:
+        x[:, 1::4] *= -1  # both zeros, one value
+    assert check(x.to(torch.bfloat16), 1) <= 1
+
+
+def test_more_rows_than_a_launch():
+    g = torch.Generator(device=DEV).manual_seed(6)
+    assert check(torch.randn(150, 4099, generator=g, device=DEV).to(torch.bfloat16), 2) <= 1
+
+
+def test_masked_and_extreme_rows():
+    g = torch.Generator(device=DEV).manual_seed(7)
+    x = torch.randn(2 * len(SETTINGS), 5000, generator=g, device=DEV)
+    x[:, 2500:] = -math.inf
+    check(x.to(torch.bfloat16), 3)
+    x = torch.full((len(SETTINGS), 5000), -math.inf, device=DEV)
+    x[:, 77] = 1.0
+    out = sample_batch(x.to(torch.bfloat16), *map(list, zip(*settings(5000))),
+                       torch.Generator(device=DEV).manual_seed(1))
+    assert out.flatten().tolist() == [77] * len(SETTINGS)
+    # greedy rows: the first of equal values, zeros of either sign, NaN largest
+    x = torch.full((3, 300), -1.0, device=DEV)
+    x[0, [40, 200]] = 2.0
+    x[1, 50], x[1, 60] = -0.0, 0.0
+    x[2, 10], x[2, [20, 30]] = 9.0, math.nan
+    out = sample_batch(x.to(torch.bfloat16), [0.0] * 3, [None] * 3, [None] * 3)
+    assert out.flatten().tolist() == [40, 50, 20]
+
+
+def test_rows_without_a_distribution_are_reported():
+    """*valid through the C ABI: a NaN, only -inf, +inf; sample_batch turns it
+    into an error as torch.multinomial does."""
+    lib = _native.lib()
+
+    def valid(fill):
+        x = torch.randn(2, 600, device=DEV).to(torch.bfloat16)
+        fill(x)
+        t, k, p = (torch.tensor(v) for v in ([0.0, 1.0], [600, 600], [1.0, 0.5]))
+        k = k.int()
+        noise = torch.rand(1, 600, device=DEV) + 0.1
+        out = torch.empty(2, dtype=torch.long, device=DEV)
+        ok = torch.empty((), dtype=torch.bool, device=DEV)
+        work = torch.empty(lib.hy_sample_workspace_bytes(2, 600), dtype=torch.uint8, device=DEV)
+        _native.check(lib.hy_sample(x.data_ptr(), 600, 0, 2, 600, t.data_ptr(), k.data_ptr(),
+                                    p.data_ptr(), noise.data_ptr(), out.data_ptr(), ok.data_ptr(),
+                                    work.data_ptr(), work.numel(),
+                                    torch.cuda.current_stream().cuda_stream), "hy_sample")
+        return bool(ok)
+
+    assert valid(lambda x: None)
+    assert valid(lambda x: x[0].fill_(math.nan))  # the greedy row
+    assert valid(lambda x: x[1, 3:].fill_(-math.inf))
+    assert not valid(lambda x: x[1, 5].fill_(math.nan))
+    assert not valid(lambda x: x[1].fill_(-math.inf))
+    assert not valid(lambda x: x[1, 9].fill_(math.inf))
