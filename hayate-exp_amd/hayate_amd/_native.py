@@ -103,6 +103,11 @@ _SIGNATURES = {
         ctypes.c_int,
     ),
     "hy_sample_workspace_bytes": ([_I32, _I32], ctypes.c_int64),
+    "hy_linear_tiles": (
+        [_P, _I64, _I32, _I32, _P, _P, _I64, _I32, _P, _I64, _P, _I64, _P, _I64, _P],
+        ctypes.c_int,
+    ),
+    "hy_linear_tiles_workspace_bytes": ([_I32, _I32, _I32, _I32], ctypes.c_int64),
     "hy_linear_add": (
         [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _I64, _P, _I64, _P],
         ctypes.c_int,

@@ -1,12 +1,13 @@
-"""The products of a decode tick's few rows with the model's weights
-(csrc/skinny.hip), and the rule that says when a module's forward may take
-them in place of its submodules' own calls.
+"""The products of a tick's rows with the model's weights (csrc/skinny.hip for
+a decode tick's few rows, csrc/tiles.hip for a prompt's many), and the rule that
+says when a module's forward may take them in place of its submodules' own calls.
 
-``norm_linear`` is RMSNorm then a projection (optionally the gated pair with
-silu), ``linear_add`` a projection plus the residual. They compute what the
-torch modules do with fp32 sums and fewer bf16 roundings, and know nothing of
-autograd, hooks or tracing: ``few_rows`` and ``plain`` hold every condition
-under which a caller must leave the modules in charge.
+For few rows ``norm_linear`` is RMSNorm then a projection (optionally the gated
+pair with silu) and ``linear_add`` a projection plus the residual; for many,
+``tile_linear`` is the gated pair or the projection plus the residual. They compute what the torch modules do with
+fp32 sums and fewer bf16 roundings, and know nothing of autograd, hooks or
+tracing: ``takes`` and ``plain`` hold every condition under which a caller must
+leave the modules in charge.
 """
 
 from __future__ import annotations
@@ -20,6 +21,7 @@ from torch.nn.modules import module as _module
 from . import _native
 
 MAX_ROWS = 32
+_MAX_STRIDE = 1 << 22
 
 
 def unwatched() -> bool:
@@ -32,14 +34,19 @@ def unwatched() -> bool:
             and c._functorch.peek_interpreter_stack() is None)
 
 
-def few_rows(x: torch.Tensor) -> bool:
-    """True when `x` (..., d) is a plain bf16 tensor of at most MAX_ROWS rows on
-    the current HIP device and nothing watches the operators run on it, nor
-    gradients or autocast change them."""
+def takes(x: torch.Tensor) -> bool:
+    """True when `x` (..., d) is a plain bf16 tensor on the current HIP device and
+    nothing watches the operators run on it, nor gradients or autocast change
+    them."""
     return (type(x) is torch.Tensor and x.dtype is torch.bfloat16 and x.is_cuda
-            and 0 < x.numel() <= MAX_ROWS * x.shape[-1]
+            and x.numel() > 0
             and not torch.is_grad_enabled() and not torch.is_autocast_enabled()
             and unwatched() and x.device.index == torch.cuda.current_device())
+
+
+def few_rows(x: torch.Tensor) -> bool:
+    """`takes`, and at most MAX_ROWS rows."""
+    return takes(x) and x.numel() <= MAX_ROWS * x.shape[-1]
 
 
 def _bare(m: nn.Module) -> bool:
@@ -52,7 +59,7 @@ def _bare(m: nn.Module) -> bool:
 def _plain_weight(w, like: torch.Tensor, dim: int) -> bool:
     return (type(w) is nn.Parameter and w.dtype is torch.bfloat16 and w.device == like.device
             and w.dim() == dim and w.stride(-1) == 1 and w.data_ptr() & 15 == 0
-            and (dim == 1 or w.stride(0) & 7 == 0))
+            and (dim == 1 or (w.stride(0) & 7 == 0 and w.stride(0) < _MAX_STRIDE)))
 
 
 def plain(x: torch.Tensor, modules=(), norms=(), linears=()) -> bool:
@@ -85,10 +92,18 @@ def add_fits(k: int, rows: int) -> bool:
     return k % 128 == 0 and k > 0 and rows <= MAX_ROWS
 
 
+def tiles_fit(k: int, n: int, rows: int) -> bool:
+    """Sizes hy_linear_tiles takes (the kernels' rows are at most _MAX_STRIDE
+    apart, which rows_of sees to for x)."""
+    return (k % 64 == 0 and n % 4 == 0 and 0 < k < _MAX_STRIDE
+            and (rows // 64 + 1) * (n // 48 + 1) < 1 << 23)
+
+
 def rows_of(x: torch.Tensor) -> torch.Tensor:
     """x (..., d) as (rows, d) with rows the kernels can read."""
     x = x.reshape(-1, x.shape[-1])
-    if x.stride(1) != 1 or x.stride(0) & 7 or x.data_ptr() & 15:
+    if (x.stride(1) != 1 or x.stride(0) & 7 or x.stride(0) >= _MAX_STRIDE
+            or x.data_ptr() & 15):
         x = x.contiguous()
         if x.data_ptr() & 15:
             x = x.clone()
@@ -123,4 +138,25 @@ def linear_add(x: torch.Tensor, weight: torch.Tensor,
         torch.cuda.current_stream(x.device).cuda_stream)
     if rc:
         _native.check(rc, "hy_linear_add")
+    return y
+
+
+def tile_linear(x: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch.Tensor] = None,
+                residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x W^T + residual, or silu(x W^T) * (x U^T); x is (rows, k), any rows."""
+    m, k = x.shape
+    n = weight.shape[0]
+    lib = _native.lib()
+    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    size = lib.hy_linear_tiles_workspace_bytes(m, n, k, up_weight is not None)
+    work = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
+    rc = lib.hy_linear_tiles(
+        x.data_ptr(), x.stride(0), m, k, weight.data_ptr(),
+        None if up_weight is None else up_weight.data_ptr(), weight.stride(0), n,
+        None if residual is None else residual.data_ptr(),
+        0 if residual is None else residual.stride(0), y.data_ptr(), n,
+        None if work is None else work.data_ptr(), size,
+        torch.cuda.current_stream(x.device).cuda_stream)
+    if rc:
+        _native.check(rc, "hy_linear_tiles")
     return y

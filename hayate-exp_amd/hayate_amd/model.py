@@ -6,8 +6,10 @@ input_layernorm, post_attention_layernorm}, norm, out_head), block.py:8-58
 and linear.py:5-22, so a checkpoint loads through the same name map
 (hayate/utils.py:114-144). Only the paged mode (the one Engine uses,
 engine.py:218-223) is provided: attention goes through
-hayate_amd.attention.GroupedQueryAttention and the HIP kernels; the
-projections, norms and the MLP stay torch ops.
+hayate_amd.attention.GroupedQueryAttention and the HIP kernels. So do the
+block's and the head's products where hayate_amd.linear takes them (bf16
+inference on the GPU with nothing watching the modules); otherwise
+projections, norms and the MLP are torch ops.
 
 The geometry is a Qwen3Config (Qwen3-4B by default, qwen.py:14-31); tests
 build smaller models with the same attention heads.
@@ -68,8 +70,11 @@ class TransformerBlock(nn.Module):
 
     def forward(self, x, cos, sin, position_ids, prev_k, prev_v, varlen_metadata=None,
                 paged_cache=None, layer_idx=None):
-        if paged_cache is not None and linear.few_rows(x) and self._few_rows_fit(x):
-            return self._few_rows(x, cos, sin, paged_cache, layer_idx), None, None
+        if paged_cache is not None and linear.takes(x) and self._plain(x):
+            if self._few_rows_fit(x):
+                return self._few_rows(x, cos, sin, paged_cache, layer_idx), None, None
+            if self._many_rows_fit(x):
+                return self._many_rows(x, cos, sin, paged_cache, layer_idx), None, None
         shortcut = x
         x, new_k, new_v = self.self_attn(self.input_layernorm(x), cos, sin, position_ids, prev_k,
                                          prev_v, varlen_metadata, paged_cache, layer_idx)
@@ -78,8 +83,8 @@ class TransformerBlock(nn.Module):
         x = self.mlp(self.post_attention_layernorm(x)) + shortcut
         return x, new_k, new_v
 
-    def _few_rows_fit(self, x) -> bool:
-        """Whether the fused path below computes what the modules would."""
+    def _plain(self, x) -> bool:
+        """Whether the fused paths below compute what the modules would."""
         attn, mlp = self.self_attn, self.mlp
         if type(attn) is not GroupedQueryAttention or type(mlp) is not FeedForward or x.dim() != 3:
             return False
@@ -89,16 +94,28 @@ class TransformerBlock(nn.Module):
                             linears=(*qkv, attn.o_proj, mlp.gate_proj, mlp.up_proj,
                                      mlp.down_proj)):
             return False
-        rows, d = x.shape[0] * x.shape[1], x.shape[2]
-        heads, mid = attn.num_heads * attn.head_dim, mlp.gate_proj.weight.shape[0]
-        return (linear.norm_fits(d, rows) and linear.add_fits(heads, rows)
-                and linear.add_fits(mid, rows)
-                and all(lin.weight.shape[1] == d for lin in qkv)
+        d, heads, mid = x.shape[2], attn.num_heads * attn.head_dim, mlp.gate_proj.weight.shape[0]
+        return (all(lin.weight.shape[1] == d for lin in qkv)
                 and attn.q_proj.weight.shape[0] == heads
                 and attn.o_proj.weight.shape == (d, heads)
                 and mlp.gate_proj.weight.shape == mlp.up_proj.weight.shape == (mid, d)
                 and mlp.gate_proj.weight.stride() == mlp.up_proj.weight.stride()
                 and mlp.down_proj.weight.shape == (d, mid))
+
+    def _few_rows_fit(self, x) -> bool:
+        """Whether the few-row kernels take these sizes: up to 32 rows they read
+        the weights at the HBM rate and fold the norms in."""
+        rows, d = x.shape[0] * x.shape[1], x.shape[2]
+        return (linear.norm_fits(d, rows)
+                and linear.add_fits(self.self_attn.o_proj.weight.shape[1], rows)
+                and linear.add_fits(self.mlp.down_proj.weight.shape[1], rows))
+
+    def _many_rows_fit(self, x) -> bool:
+        """Whether the tile kernels take these sizes (any number of rows)."""
+        rows, d = x.shape[0] * x.shape[1], x.shape[2]
+        heads, mid = self.self_attn.o_proj.weight.shape[1], self.mlp.down_proj.weight.shape[1]
+        return (linear.tiles_fit(heads, d, rows) and linear.tiles_fit(d, mid, rows)
+                and linear.tiles_fit(mid, d, rows))
 
     def _few_rows(self, x, cos, sin, paged_cache, layer_idx):
         """The block for a decode tick's few rows: norms, silu and residuals
@@ -116,6 +133,19 @@ class TransformerBlock(nn.Module):
         h = linear.norm_linear(x, norm.weight, _norm_eps(norm, x.dtype), mlp.gate_proj.weight,
                                mlp.up_proj.weight)
         return linear.linear_add(h, mlp.down_proj.weight, x).view(shape)
+
+    def _many_rows(self, x, cos, sin, paged_cache, layer_idx):
+        """The block for a prompt's rows: silu, the gating product and the
+        residuals inside the products. The q/k/v projection has nothing to
+        fuse and stays with the library."""
+        attn, mlp, shape = self.self_attn, self.mlp, x.shape
+        context = attn.context(*attn.project_qkv(self.input_layernorm(x)), cos, sin, paged_cache,
+                               layer_idx)
+        x = linear.tile_linear(linear.rows_of(context), attn.o_proj.weight,
+                               residual=linear.rows_of(x))
+        h = linear.tile_linear(self.post_attention_layernorm(x), mlp.gate_proj.weight,
+                               mlp.up_proj.weight)
+        return linear.tile_linear(h, mlp.down_proj.weight, residual=x).view(shape)
 
 
 class Qwen3Model(nn.Module):

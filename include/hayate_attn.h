@@ -370,6 +370,23 @@ int hy_linear_add(const void *x, int64_t x_stride, int32_t m, int32_t k,
                   int64_t y_stride, void *stream);
 
 /*
+ * The same products for a prompt's rows, any m: y = x W^T + residual (residual
+ * may be NULL), or with up_weight (same shape and stride as weight; residual NULL)
+ * y = silu(x W^T) * (x up_weight^T). fp32 sums, one rounding. k is a multiple of
+ * 64, n of 4, strides below 2^22 elements; other sizes return HY_EUNSUPPORTED.
+ * workspace is device memory of hy_linear_tiles_workspace_bytes(m, n, k, gated)
+ * bytes, 16-byte aligned (NULL when that is 0).
+ * Replaces o_proj and down_proj with the residual additions of
+ * hayate/model/block.py:45-58 and gate_proj, up_proj and silu (linear.py:18-22).
+ */
+int64_t hy_linear_tiles_workspace_bytes(int32_t m, int32_t n, int32_t k, int32_t gated);
+int hy_linear_tiles(const void *x, int64_t x_stride, int32_t m, int32_t k,
+                    const void *weight, const void *up_weight, int64_t w_stride,
+                    int32_t n, const void *residual, int64_t r_stride, void *y,
+                    int64_t y_stride, void *workspace, int64_t workspace_bytes,
+                    void *stream);
+
+/*
  * One token per row of 16-bit logits (dtype 0: bf16, 1: fp16; rows row_stride
  * apart, values contiguous). temperature, top_k and top_p are host arrays of
  * n_rows entries, read before the call returns. temperature 0: the first
