@@ -30,13 +30,14 @@ qkv_rebuilds = 0
 
 def _views_of(f: torch.Tensor, ws) -> bool:
     """True when `ws` are consecutive row blocks of `f`, in order."""
-    row = 0
+    row, at = 0, f.data_ptr()
+    stride, columns, dtype, device = f.stride(), f.shape[1:], f.dtype, f.device
+    row_bytes = stride[0] * f.element_size()
     for w in ws:
-        n = w.shape[0]
-        if (w.device != f.device or w.dtype != f.dtype or w.shape[1:] != f.shape[1:]
-                or w.stride() != f.stride() or w.data_ptr() != f[row : row + n].data_ptr()):
+        if (w.data_ptr() != at + row * row_bytes or w.dtype is not dtype or w.stride() != stride
+                or w.shape[1:] != columns or w.device != device):
             return False
-        row += n
+        row += w.shape[0]
     return row == f.shape[0]
 
 
@@ -72,7 +73,8 @@ class GroupedQueryAttention(nn.Module):
         `qkv_rebuilds`, so holders of its address (captured graphs) can
         tell."""
         global qkv_rebuilds
-        lins = (self.q_proj, self.k_proj, self.v_proj)
+        mods = self._modules
+        lins = (mods["q_proj"], mods["k_proj"], mods["v_proj"])
         f = self._qkv_weight
         if f is not None and _views_of(f, [lin.weight for lin in lins]):
             return f
@@ -96,13 +98,10 @@ class GroupedQueryAttention(nn.Module):
 
     def split_qkv(self, y):
         """The q, k and v views of a fused projection's output (B, T, rows)."""
-        B, T, _ = y.shape
-        hq = self.num_heads * self.head_dim
-        hkv = self.num_kv_groups * self.head_dim
-        q = y[..., :hq].view(B, T, self.num_heads, self.head_dim)
-        k = y[..., hq : hq + hkv].view(B, T, self.num_kv_groups, self.head_dim)
-        v = y[..., hq + hkv :].view(B, T, self.num_kv_groups, self.head_dim)
-        return q, k, v
+        B, T, rows = y.shape
+        hq, hkv = self.num_heads, self.num_kv_groups
+        heads = y.view(B, T, hq + 2 * hkv, self.head_dim)
+        return heads.narrow(2, 0, hq), heads.narrow(2, hq, hkv), heads.narrow(2, hq + hkv, hkv)
 
     def forward(
         self,
@@ -132,17 +131,17 @@ class GroupedQueryAttention(nn.Module):
         """Norm, rope, append and paged attention of projected q, k, v (B, T,
         H, D): the input of o_proj, (B, T, Hq * D)."""
         B, T = q.shape[:2]
-        q_norm_w = self.q_norm.weight
-        k_norm_w = self.k_norm.weight
+        q_norm, k_norm = self.q_norm, self.k_norm
+        q_norm_w, k_norm_w = q_norm.weight, k_norm.weight
         # each norm keeps its own eps; None means the input dtype's epsilon,
         # as nn.RMSNorm resolves it
-        eps = _norm_eps(self.q_norm, q.dtype)
-        k_eps = _norm_eps(self.k_norm, k.dtype)
+        eps = _norm_eps(q_norm, q.dtype)
+        k_eps = _norm_eps(k_norm, k.dtype)
         if paged_cache.varlen:
             # Varlen ticks carry packed tokens: x is (1, N, d_in).
             if B != 1:
                 raise ValueError("a varlen tick expects x of shape (1, tokens, d_in)")
-            if all(ql == 1 for ql in paged_cache.q_lens):
+            if paged_cache.decode_only:
                 # a decode tick: norm, rope, append and attention in one launch
                 _, context = paged_cache.decode_layer(
                     layer_idx, q[0], k[0], v[0], q_norm_w, k_norm_w, eps, cos, sin,

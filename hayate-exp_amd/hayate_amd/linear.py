@@ -22,6 +22,7 @@ from . import _native
 
 MAX_ROWS = 32
 _MAX_STRIDE = 1 << 22
+_Parameter, _Linear, _RMSNorm = nn.Parameter, nn.Linear, nn.RMSNorm
 
 
 def unwatched() -> bool:
@@ -56,10 +57,13 @@ def _bare(m: nn.Module) -> bool:
                 or d["_backward_pre_hooks"] or "forward" in d)
 
 
-def _plain_weight(w, like: torch.Tensor, dim: int) -> bool:
-    return (type(w) is nn.Parameter and w.dtype is torch.bfloat16 and w.device == like.device
-            and w.dim() == dim and w.stride(-1) == 1 and w.data_ptr() & 15 == 0
-            and (dim == 1 or (w.stride(0) & 7 == 0 and w.stride(0) < _MAX_STRIDE)))
+def _plain_weight(w, device_index: int, dim: int) -> bool:
+    if (type(w) is not _Parameter or w.dtype is not torch.bfloat16
+            or w.get_device() != device_index):
+        return False
+    st = w.stride()
+    return (len(st) == dim and st[-1] == 1 and w.data_ptr() & 15 == 0
+            and (dim == 1 or (st[0] & 7 == 0 and st[0] < _MAX_STRIDE)))
 
 
 def plain(x: torch.Tensor, modules=(), norms=(), linears=()) -> bool:
@@ -68,16 +72,19 @@ def plain(x: torch.Tensor, modules=(), norms=(), linears=()) -> bool:
     kernels can read."""
     if _module._has_any_global_hook():
         return False
+    index, shape = x.get_device(), (x.shape[-1],)
     for m in modules:
         if not _bare(m):
             return False
     for m in norms:
-        if not (type(m) is nn.RMSNorm and _bare(m) and m.normalized_shape == (x.shape[-1],)
-                and _plain_weight(m._parameters.get("weight"), x, 1)):
+        if not (type(m) is _RMSNorm and _bare(m) and m.normalized_shape == shape
+                and _plain_weight(m._parameters.get("weight"), index, 1)):
             return False
     for m in linears:
-        if not (type(m) is nn.Linear and _bare(m) and m._parameters.get("bias") is None
-                and _plain_weight(m._parameters.get("weight"), x, 2)):
+        if type(m) is not _Linear or not _bare(m):
+            return False
+        p = m._parameters
+        if p.get("bias") is not None or not _plain_weight(p.get("weight"), index, 2):
             return False
     return True
 
@@ -115,11 +122,11 @@ def norm_linear(x: torch.Tensor, norm_weight: Optional[torch.Tensor], eps: float
     """norm(x) W^T, or silu(norm(x) W^T) * (norm(x) U^T); x is (rows, k)."""
     m, k = x.shape
     n = weight.shape[0]
-    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    y = x.new_empty((m, n))
     rc = _native.lib().hy_norm_linear(
         x.data_ptr(), x.stride(0), m, k, None if norm_weight is None else norm_weight.data_ptr(),
         eps, weight.data_ptr(), None if up_weight is None else up_weight.data_ptr(),
-        weight.stride(0), n, y.data_ptr(), n, torch.cuda.current_stream(x.device).cuda_stream)
+        weight.stride(0), n, y.data_ptr(), n, _native.stream_of(x.get_device()))
     if rc:
         _native.check(rc, "hy_norm_linear")
     return y
@@ -130,12 +137,12 @@ def linear_add(x: torch.Tensor, weight: torch.Tensor,
     """x W^T + residual; x is (rows, k)."""
     m, k = x.shape
     n = weight.shape[0]
-    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    y = x.new_empty((m, n))
     rc = _native.lib().hy_linear_add(
         x.data_ptr(), x.stride(0), m, k, weight.data_ptr(), weight.stride(0), n,
         None if residual is None else residual.data_ptr(),
         0 if residual is None else residual.stride(0), y.data_ptr(), n,
-        torch.cuda.current_stream(x.device).cuda_stream)
+        _native.stream_of(x.get_device()))
     if rc:
         _native.check(rc, "hy_linear_add")
     return y
@@ -147,7 +154,7 @@ def tile_linear(x: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch
     m, k = x.shape
     n = weight.shape[0]
     lib = _native.lib()
-    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    y = x.new_empty((m, n))
     size = lib.hy_linear_tiles_workspace_bytes(m, n, k, up_weight is not None)
     work = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
     rc = lib.hy_linear_tiles(
@@ -156,7 +163,7 @@ def tile_linear(x: torch.Tensor, weight: torch.Tensor, up_weight: Optional[torch
         None if residual is None else residual.data_ptr(),
         0 if residual is None else residual.stride(0), y.data_ptr(), n,
         None if work is None else work.data_ptr(), size,
-        torch.cuda.current_stream(x.device).cuda_stream)
+        _native.stream_of(x.get_device()))
     if rc:
         _native.check(rc, "hy_linear_tiles")
     return y

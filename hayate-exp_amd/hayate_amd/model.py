@@ -18,6 +18,7 @@ build smaller models with the same attention heads.
 from __future__ import annotations
 
 from dataclasses import dataclass
+from typing import NamedTuple
 
 import torch
 import torch.nn as nn
@@ -41,6 +42,18 @@ class Qwen3Config:
     rms_norm_eps: float = 1e-6
     rope_theta: int = 1_000_000
     max_position_embeddings: int = 40_960
+
+
+class _Weights(NamedTuple):
+    """What a block's fused paths read (the q, k and v weights are the
+    attention module's fused buffer)."""
+
+    in_norm: nn.RMSNorm
+    post_norm: nn.RMSNorm
+    o: torch.Tensor
+    gate: torch.Tensor
+    up: torch.Tensor
+    down: torch.Tensor
 
 
 class FeedForward(nn.Module):
@@ -70,11 +83,18 @@ class TransformerBlock(nn.Module):
 
     def forward(self, x, cos, sin, position_ids, prev_k, prev_v, varlen_metadata=None,
                 paged_cache=None, layer_idx=None):
-        if paged_cache is not None and linear.takes(x) and self._plain(x):
-            if self._few_rows_fit(x):
-                return self._few_rows(x, cos, sin, paged_cache, layer_idx), None, None
-            if self._many_rows_fit(x):
-                return self._many_rows(x, cos, sin, paged_cache, layer_idx), None, None
+        if paged_cache is not None and linear.takes(x):
+            w = self._plain_weights(x)
+            if w is not None:
+                rows, (d, heads), mid = x.shape[0] * x.shape[1], w.o.shape, w.down.shape[1]
+                # up to 32 rows the few-row kernels, which read the weights at the
+                # HBM rate and fold the norms in; tiles take any number
+                if (linear.norm_fits(d, rows) and linear.add_fits(heads, rows)
+                        and linear.add_fits(mid, rows)):
+                    return self._few_rows(x, w, cos, sin, paged_cache, layer_idx), None, None
+                if (linear.tiles_fit(heads, d, rows) and linear.tiles_fit(d, mid, rows)
+                        and linear.tiles_fit(mid, d, rows)):
+                    return self._many_rows(x, w, cos, sin, paged_cache, layer_idx), None, None
         shortcut = x
         x, new_k, new_v = self.self_attn(self.input_layernorm(x), cos, sin, position_ids, prev_k,
                                          prev_v, varlen_metadata, paged_cache, layer_idx)
@@ -83,69 +103,53 @@ class TransformerBlock(nn.Module):
         x = self.mlp(self.post_attention_layernorm(x)) + shortcut
         return x, new_k, new_v
 
-    def _plain(self, x) -> bool:
-        """Whether the fused paths below compute what the modules would."""
-        attn, mlp = self.self_attn, self.mlp
+    def _plain_weights(self, x):
+        """The weights of the fused paths below, when those compute what the
+        modules would, else None."""
+        mods = self._modules
+        attn, mlp = mods.get("self_attn"), mods.get("mlp")
         if type(attn) is not GroupedQueryAttention or type(mlp) is not FeedForward or x.dim() != 3:
-            return False
-        qkv = (attn.q_proj, attn.k_proj, attn.v_proj)
-        if not linear.plain(x, modules=(attn, mlp),
-                            norms=(self.input_layernorm, self.post_attention_layernorm),
-                            linears=(*qkv, attn.o_proj, mlp.gate_proj, mlp.up_proj,
-                                     mlp.down_proj)):
-            return False
-        d, heads, mid = x.shape[2], attn.num_heads * attn.head_dim, mlp.gate_proj.weight.shape[0]
-        return (all(lin.weight.shape[1] == d for lin in qkv)
-                and attn.q_proj.weight.shape[0] == heads
-                and attn.o_proj.weight.shape == (d, heads)
-                and mlp.gate_proj.weight.shape == mlp.up_proj.weight.shape == (mid, d)
-                and mlp.gate_proj.weight.stride() == mlp.up_proj.weight.stride()
-                and mlp.down_proj.weight.shape == (d, mid))
+            return None
+        # straight from the modules' tables: nn.Module's attribute lookup takes
+        # about 0.5 us a name, and this runs for every layer of every tick
+        a, f = attn._modules, mlp._modules
+        norms = in_norm, post_norm = mods.get("input_layernorm"), mods.get("post_attention_layernorm")
+        linears = [a.get("q_proj"), a.get("k_proj"), a.get("v_proj"), a.get("o_proj"),
+                   f.get("gate_proj"), f.get("up_proj"), f.get("down_proj")]
+        if not linear.plain(x, modules=(attn, mlp), norms=norms, linears=linears):
+            return None
+        q, k, v, o, gate, up, down = [m._parameters["weight"] for m in linears]
+        d, heads, shape = x.shape[2], attn.num_heads * attn.head_dim, gate.shape
+        if (q.shape != (heads, d) or k.shape[1] != d or v.shape[1] != d or o.shape != (d, heads)
+                or shape[1] != d or up.shape != shape or up.stride() != gate.stride()
+                or down.shape != (d, shape[0])):
+            return None
+        return _Weights(in_norm, post_norm, o, gate, up, down)
 
-    def _few_rows_fit(self, x) -> bool:
-        """Whether the few-row kernels take these sizes: up to 32 rows they read
-        the weights at the HBM rate and fold the norms in."""
-        rows, d = x.shape[0] * x.shape[1], x.shape[2]
-        return (linear.norm_fits(d, rows)
-                and linear.add_fits(self.self_attn.o_proj.weight.shape[1], rows)
-                and linear.add_fits(self.mlp.down_proj.weight.shape[1], rows))
-
-    def _many_rows_fit(self, x) -> bool:
-        """Whether the tile kernels take these sizes (any number of rows)."""
-        rows, d = x.shape[0] * x.shape[1], x.shape[2]
-        heads, mid = self.self_attn.o_proj.weight.shape[1], self.mlp.down_proj.weight.shape[1]
-        return (linear.tiles_fit(heads, d, rows) and linear.tiles_fit(d, mid, rows)
-                and linear.tiles_fit(mid, d, rows))
-
-    def _few_rows(self, x, cos, sin, paged_cache, layer_idx):
+    def _few_rows(self, x, w, cos, sin, paged_cache, layer_idx):
         """The block for a decode tick's few rows: norms, silu and residuals
         inside the four products, two launches beside the attention's own per
         half of the block."""
-        attn, mlp, shape = self.self_attn, self.mlp, x.shape
-        norm = self.input_layernorm
+        attn, shape = self._modules["self_attn"], x.shape
         x = linear.rows_of(x)
-        qkv = linear.norm_linear(x, norm.weight, _norm_eps(norm, x.dtype),
-                                 attn.fused_qkv_weight())
-        context = attn.context(*attn.split_qkv(qkv.view(*shape[:2], -1)), cos, sin, paged_cache,
-                               layer_idx)
-        x = linear.linear_add(linear.rows_of(context), attn.o_proj.weight, x)
-        norm = self.post_attention_layernorm
-        h = linear.norm_linear(x, norm.weight, _norm_eps(norm, x.dtype), mlp.gate_proj.weight,
-                               mlp.up_proj.weight)
-        return linear.linear_add(h, mlp.down_proj.weight, x).view(shape)
+        qkv = linear.norm_linear(x, w.in_norm._parameters["weight"],
+                                 _norm_eps(w.in_norm, x.dtype), attn.fused_qkv_weight())
+        context = attn.context(*attn.split_qkv(qkv.view(shape[0], shape[1], -1)), cos, sin,
+                               paged_cache, layer_idx)
+        x = linear.linear_add(linear.rows_of(context), w.o, x)
+        h = linear.norm_linear(x, w.post_norm._parameters["weight"],
+                               _norm_eps(w.post_norm, x.dtype), w.gate, w.up)
+        return linear.linear_add(h, w.down, x).view(shape)
 
-    def _many_rows(self, x, cos, sin, paged_cache, layer_idx):
+    def _many_rows(self, x, w, cos, sin, paged_cache, layer_idx):
         """The block for a prompt's rows: silu, the gating product and the
         residuals inside the products. The q/k/v projection has nothing to
         fuse and stays with the library."""
-        attn, mlp, shape = self.self_attn, self.mlp, x.shape
-        context = attn.context(*attn.project_qkv(self.input_layernorm(x)), cos, sin, paged_cache,
-                               layer_idx)
-        x = linear.tile_linear(linear.rows_of(context), attn.o_proj.weight,
-                               residual=linear.rows_of(x))
-        h = linear.tile_linear(self.post_attention_layernorm(x), mlp.gate_proj.weight,
-                               mlp.up_proj.weight)
-        return linear.tile_linear(h, mlp.down_proj.weight, residual=x).view(shape)
+        attn, shape = self._modules["self_attn"], x.shape
+        context = attn.context(*attn.project_qkv(w.in_norm(x)), cos, sin, paged_cache, layer_idx)
+        x = linear.tile_linear(linear.rows_of(context), w.o, residual=linear.rows_of(x))
+        h = linear.tile_linear(w.post_norm(x), w.gate, w.up)
+        return linear.tile_linear(h, w.down, residual=x).view(shape)
 
 
 class Qwen3Model(nn.Module):

@@ -102,7 +102,8 @@ class PagedPrefix:
 
 
 def _stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return _native.stream_of(torch.cuda.current_device() if device.index is None
+                             else device.index)
 
 
 def _require_hip(t: torch.Tensor, what: str) -> None:
@@ -234,6 +235,7 @@ class PagedKVBatch:
         self.head_dim = manager.head_dim
         self.varlen = varlen
         self.q_lens = list(q_lens)
+        self.decode_only = all(q == 1 for q in self.q_lens)
         self.cache_lens_host = list(cache_lens_host)
         self.kv_lens_host = [c + q for c, q in zip(cache_lens_host, q_lens)]
         self.num_seqs = len(q_lens)
@@ -455,7 +457,7 @@ class PagedKVBatch:
         hy_paged_decode_append_noalloc, whose partials live in the library's
         static device scratch instead of the plan's workspace (same
         results; raises MemoryError if the tick's partials do not fit)."""
-        if any(ql != 1 for ql in self.q_lens):
+        if not self.decode_only:
             raise ValueError("decode_layer needs q_len == 1 for every sequence")
         a = self._append_inputs("decode_layer", q, k, v, q_norm_weight, k_norm_weight, cos,
                                 sin)

@@ -121,6 +121,7 @@ class StaticTickBatch(PagedKVBatch):
         self.varlen = True
         self.q_lens = q_lens
         self.num_seqs = B
+        self.decode_only = all(q == 1 for q in q_lens)
         self.total_tokens = sum(q_lens)
         self.query_len = None
         self.tokens_per_split = manager.tokens_per_split
