@@ -109,6 +109,7 @@ _SIGNATURES = {
         ctypes.c_int,
     ),
     "hy_linear_tiles_workspace_bytes": ([_I32, _I32, _I32, _I32], ctypes.c_int64),
+    "hy_row_norm": ([_P, _I64, _I32, _I32, _P, _F32, _P, _P], ctypes.c_int),
     "hy_linear_add": (
         [_P, _I64, _I32, _I32, _P, _I64, _I32, _P, _I64, _P, _I64, _P],
         ctypes.c_int,

@@ -4,7 +4,8 @@ says when a module's forward may take them in place of its submodules' own calls
 
 For few rows ``norm_linear`` is RMSNorm then a projection (optionally the gated
 pair with silu) and ``linear_add`` a projection plus the residual; for many,
-``tile_linear`` is the gated pair or the projection plus the residual. They compute what the torch modules do with
+``row_norm`` is the norm and ``tile_linear`` the gated pair or the projection
+plus the residual. They compute what the torch modules do with
 fp32 sums and fewer bf16 roundings, and know nothing of autograd, hooks or
 tracing: ``takes`` and ``plain`` hold every condition under which a caller must
 leave the modules in charge.
@@ -106,6 +107,11 @@ def tiles_fit(k: int, n: int, rows: int) -> bool:
             and (rows // 64 + 1) * (n // 48 + 1) < 1 << 23)
 
 
+def row_norm_fits(k: int) -> bool:
+    """Sizes hy_row_norm takes."""
+    return k % 8 == 0 and 0 < k <= 4096
+
+
 def rows_of(x: torch.Tensor) -> torch.Tensor:
     """x (..., d) as (rows, d) with rows the kernels can read."""
     x = x.reshape(-1, x.shape[-1])
@@ -145,6 +151,17 @@ def linear_add(x: torch.Tensor, weight: torch.Tensor,
         _native.stream_of(x.get_device()))
     if rc:
         _native.check(rc, "hy_linear_add")
+    return y
+
+
+def row_norm(x: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """RMSNorm of x (rows, k)."""
+    m, k = x.shape
+    y = x.new_empty((m, k))
+    rc = _native.lib().hy_row_norm(x.data_ptr(), x.stride(0), m, k, norm_weight.data_ptr(), eps,
+                                   y.data_ptr(), _native.stream_of(x.get_device()))
+    if rc:
+        _native.check(rc, "hy_row_norm")
     return y
 
 

@@ -92,8 +92,8 @@ class TransformerBlock(nn.Module):
                 if (linear.norm_fits(d, rows) and linear.add_fits(heads, rows)
                         and linear.add_fits(mid, rows)):
                     return self._few_rows(x, w, cos, sin, paged_cache, layer_idx), None, None
-                if (linear.tiles_fit(heads, d, rows) and linear.tiles_fit(d, mid, rows)
-                        and linear.tiles_fit(mid, d, rows)):
+                if (linear.row_norm_fits(d) and linear.tiles_fit(heads, d, rows)
+                        and linear.tiles_fit(d, mid, rows) and linear.tiles_fit(mid, d, rows)):
                     return self._many_rows(x, w, cos, sin, paged_cache, layer_idx), None, None
         shortcut = x
         x, new_k, new_v = self.self_attn(self.input_layernorm(x), cos, sin, position_ids, prev_k,
@@ -146,9 +146,12 @@ class TransformerBlock(nn.Module):
         residuals inside the products. The q/k/v projection has nothing to
         fuse and stays with the library."""
         attn, shape = self._modules["self_attn"], x.shape
-        context = attn.context(*attn.project_qkv(w.in_norm(x)), cos, sin, paged_cache, layer_idx)
-        x = linear.tile_linear(linear.rows_of(context), w.o, residual=linear.rows_of(x))
-        h = linear.tile_linear(w.post_norm(x), w.gate, w.up)
+        x = linear.rows_of(x)
+        h = linear.row_norm(x, w.in_norm._parameters["weight"], _norm_eps(w.in_norm, x.dtype))
+        context = attn.context(*attn.project_qkv(h.view(shape)), cos, sin, paged_cache, layer_idx)
+        x = linear.tile_linear(linear.rows_of(context), w.o, residual=x)
+        h = linear.row_norm(x, w.post_norm._parameters["weight"], _norm_eps(w.post_norm, x.dtype))
+        h = linear.tile_linear(h, w.gate, w.up)
         return linear.tile_linear(h, w.down, residual=x).view(shape)
 
 

@@ -387,6 +387,15 @@ int hy_linear_tiles(const void *x, int64_t x_stride, int32_t m, int32_t k,
                     void *stream);
 
 /*
+ * RMSNorm of bf16 rows: y[m][k] (rows contiguous) = (x / sqrt(mean(x^2) + eps)) *
+ * norm_weight in fp32, one rounding. k is a multiple of 8 up to 4096; other sizes
+ * return HY_EUNSUPPORTED. Replaces input_layernorm and post_attention_layernorm
+ * (hayate/model/block.py:33-58) for a prompt's rows.
+ */
+int hy_row_norm(const void *x, int64_t x_stride, int32_t m, int32_t k,
+                const void *norm_weight, float eps, void *y, void *stream);
+
+/*
  * One token per row of 16-bit logits (dtype 0: bf16, 1: fp16; rows row_stride
  * apart, values contiguous). temperature, top_k and top_p are host arrays of
  * n_rows entries, read before the call returns. temperature 0: the first

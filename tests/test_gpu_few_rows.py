@@ -3,7 +3,7 @@
 The products against float64 at the sizes where the kernels change shape:
 row counts around the 16-row tiles, column counts that leave a workgroup a
 partial tile or nothing, and K around the waves' step counts. The result is
-rounded to bf16 once (at most 2^-9 of each value) and, with the norm, each
+rounded to bf16 once (at most 2^-8 of each value) and, with the norm, each
 x * weight before the sums: those errors are independent, so a sum of them
 is below 2^-8 of the root of its terms' sum of squares (three standard
 deviations), of which a sum that cancels is only a part.
@@ -141,7 +141,7 @@ def test_block_equals_its_modules(q_lens, monkeypatch):
         assert len(used) == (2 if sum(q_lens) <= 32 else 0)
     e = rel(fused, plain.double())
     say(f"  relative difference {e:.2e}")
-    # five rounded products on either side, each 2^-9 of a part of the sum
+    # five rounded products on either side, each 2^-8 of a part of the sum
     assert e < 2**-7
     assert rel(k1, m.k_cache.double()) < 2**-8
 

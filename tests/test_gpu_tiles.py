@@ -3,7 +3,7 @@
 Against float64 at the sizes where the plan changes: every tile shape, split
 and whole, row and column counts that leave the last tile one row, all but
 one, or a fraction of a fragment, and K of one step, of fewer steps than the
-ring has stages and of many. The result is rounded to bf16 once (at most 2^-9
+ring has stages and of many. The result is rounded to bf16 once (at most 2^-8
 of each value); the fp32 sums add far less.
 """
 
@@ -55,6 +55,18 @@ def test_gated_linear(m, n, k):
     gate = x.double() @ w.double().T
     exact = gate * torch.sigmoid(gate) * (x.double() @ u.double().T)
     assert rel(linear.tile_linear(x, w, u), exact) < 2**-8
+
+
+@pytest.mark.parametrize("k", [8, 504, 512, 520, 2560, 3592, 4096])
+@pytest.mark.parametrize("m", [1, 33, 4096, 4099])
+def test_row_norm(m, k):
+    """fp32 sums of k squares, one rounding to bf16 (8 significant bits)."""
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    wide = bf16(g, m, k + 8, std=3.0)
+    x, w = wide[:, :k], 1 + bf16(g, k, std=0.2)
+    exact = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-3) * w.double()
+    y = linear.row_norm(x, w, 1e-3).double()
+    assert ((y - exact).abs() <= (2**-8 + 1e-5) * exact.abs() + 1e-30).all()
 
 
 def test_nothing_outside_the_result_is_written():
@@ -112,5 +124,5 @@ def test_block_equals_its_modules(lens):
             outs.append(block(x, cos, sin, None, None, None, None, batch, 0)[0])
         if hook:
             hook.remove()
-    # five roundings of 2^-9 in a chain of products at most
+    # five roundings of 2^-8 in a chain of products at most
     assert rel(outs[0], outs[1].double()) < 5 * 2**-8
