@@ -45,6 +45,9 @@ constexpr int kPrefillKeys = hy::kPrefillTileKeys;  // keys per prefill step
 // 6.4 us (3.4 steps) after the previous one's last step; the merge launch
 // costs about two steps and one split partial (write + read of its rows of
 // fp32 O) a fortieth of a step.
+// The prologue and epilogue have since lost about 2 us; settings of 1.4-2.9
+// fixed, 1.9-3.4 gap and 1.2-2.0 for the merge stay within 1 % of each other on
+// eleven prompt and mixed ticks, so these were kept.
 constexpr double kPrefillFixed = 2.9;
 constexpr double kPrefillGap = 3.4;
 constexpr double kMergeLaunch = 2.0;

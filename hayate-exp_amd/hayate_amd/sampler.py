@@ -13,7 +13,7 @@ The reference loops over rows in Python, one small kernel chain per row
 (:67-85). Here every row of the batch goes through one sort and a handful of
 batched ops, with per-row temperature / k / p as tensors, so a tick costs
 the same few launches whatever the batch size. 16-bit logits on a HIP device
-(the engine's) take hy_sample instead: one launch, no sort, the same draws
+(the engine's) take hy_sample instead: no sort, the same draws
 from the same generator.
 """
 
