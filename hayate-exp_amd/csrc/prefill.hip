@@ -32,7 +32,7 @@
 // gfx950's 16-byte direct-to-LDS loads (global_load_lds_dwordx4), two tiles
 // ahead of the one being consumed, without passing through registers; one
 // wait and one barrier per tile. The fourth stage keeps a tile's V rows in
-// place while the next tile's first block runs their P V (below). A load
+// place while the next tile's first block runs their P V (below, G >= 4). A load
 // instruction writes 64 lanes x 16 bytes to consecutive LDS addresses, so
 // the bank-conflict-free layouts are lane permutations instead of padded rows.
 // Four neighbouring lanes must stay within 64 bytes of one row: with lanes
@@ -207,6 +207,15 @@ void prefill_kernel(
   const int r = 32 * wave + c;
   const int row_tok = q_begin + r / G;
   const bool live = row_tok < q_end;
+  // Whether a block's P V runs in the next block's body (see the pipeline
+  // below), the last block's after the loop. That leaves a stage only one
+  // tile behind the barrier to be read, which holds while the item's tokens
+  // (kRows / G) span no more than a tile: with fewer heads a wave's last
+  // block can lie four tiles before the item's last (G = 1) or two (G = 2),
+  // in a stage that by then holds another tile or the epilogue's rows. P V in
+  // the own body costs those 0-1 % (G = 2: 4 x 512 at offsets 0-3584 54.2
+  // against 53.7 us, 8 x 512 85.2 against 84.6).
+  constexpr bool kLatePv = kRows / G <= kTile;
   bf16x8 qop[8];  // this lane's row of Q^T (zeros for rows past the chunk)
   f32x16 acc[4];
 #pragma unroll
@@ -306,7 +315,8 @@ void prefill_kernel(
 
   // Software pipeline over this wave's blocks. Block j's body runs the
   // QK^T MFMAs of block j + 1 while the VALU does block j's softmax (the
-  // two are independent), then block j - 1's P V MFMAs, so a block's
+  // two are independent), then block j - 1's P V MFMAs (or, without kLatePv,
+  // block j's after its rebase), so a block's
   // probabilities are used one body after they are made; K operands are
   // read two blocks ahead and V operands at the start of the body that
   // uses them, so no LDS read is waited for right after it is issued. The
@@ -314,7 +324,8 @@ void prefill_kernel(
   // the softmax runs; block j - 1's P V goes in before block j's rebase,
   // which then scales it with the rest of the accumulator. Measured against
   // P V in the block's own body: 0.5 % less on prefill_4x512 and 0.7 % on
-  // the mixed tick (graph steps, alternating runs).
+  // the mixed tick (graph steps, alternating runs). Either order updates the
+  // accumulators with the same operations.
   bf16x8 kop[8];
   auto read_k = [&](int j) __attribute__((always_inline)) {
     const uint16_t *kb = k_block(j);
@@ -419,7 +430,7 @@ void prefill_kernel(
             __builtin_bit_cast(bf16x8, vop[2 * db + kh2]), kh2 ? pop1 : pop0, acc[db], 0, 0, 0);
   };
 
-  // One block: half of block j - 1's V reads go out first (the LDS counter
+  // One block (with kLatePv): half of block j - 1's V reads go out first (the LDS counter
   // holds at most 15 outstanding reads, so the first MFMA's wait for the K
   // operands cannot leave all 16 in flight); then QK^T of block j + 1 on the
   // matrix core, interleaved with the other V reads and block j's
@@ -433,9 +444,9 @@ void prefill_kernel(
                   const bf16x8 &prev0, const bf16x8 &prev1) __attribute__((always_inline)) {
     float psum;
     if (masked) mask(s_cur, kv_begin + 32 * j);  // blocks on the diagonal
-    // block j - 1's V (its P V runs in this body); for j = 0 block 0's
-    // stage is read and the values are unused
-    const int jv = j > 0 ? j - 1 : 0;
+    // V of the block whose P V runs in this body; for j = 0 with kLatePv
+    // block 0's stage is read and the values are unused
+    const int jv = kLatePv ? (j > 0 ? j - 1 : 0) : j;
     read_v(jv, 0);
     __builtin_amdgcn_sched_barrier(0);
     // The two waves of a SIMD take turns: the one in this region (next
@@ -458,8 +469,9 @@ void prefill_kernel(
     __asm__ volatile("" ::"v"(psum), "v"(pop0), "v"(pop1));
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(0);
-    if (j > 0) pv(prev0, prev1);  // block j - 1's P V, before block j's rebase
+    if (kLatePv && j > 0) pv(prev0, prev1);  // block j - 1's, before block j's rebase
     rebase(s_cur, pop0, pop1, psum);
+    if (!kLatePv) pv(pop0, pop1);
     read_k(j + 2);
   };
 
@@ -522,9 +534,9 @@ void prefill_kernel(
     }
   }
 
-  // the last block's P V (its tile is still in the ring: nothing is issued
-  // after the last barrier)
-  if (nb > 0) {
+  // the last block's P V (its tile, the item's last or the one before, is
+  // still in the ring: nothing is issued after the last barrier)
+  if (kLatePv && nb > 0) {
     read_v(nb - 1, 0);
     read_v(nb - 1, 1);
     if ((nb - 1) & 1)
@@ -538,7 +550,9 @@ void prefill_kernel(
     // The output rows go through LDS so that 16 lanes store a row: a lane
     // holds 8-byte pieces of one row, and 64 lanes storing to 32 rows keep a
     // CU's memory pipe busy four times as long. The two stages after the last
-    // tile's are free (their tiles were left before the last barrier); 8 KiB
+    // tile's are free: after the last barrier only the last tile and the one
+    // before are read (other waves' K reads past their last block get the rows
+    // written here, and drop what they make of them); 8 KiB
     // a wave, 16-byte units with unit(row, chunk) = row * 16 + (chunk ^ row % 16).
     // With the partials below: a 512-token chunk 24.0 -> 21.9 us, 20 of them
     // 137 -> 125 us, 4 x 512 at offsets 0-3584 94.3 -> 93.0 us (graph steps).

@@ -1,11 +1,14 @@
 """hy_paged_prefill through the C ABI with query and output rows off 16-byte
 boundaries: the same bits as with aligned rows, for whole tiles, a chunk that
-ends inside a tile, split key ranges, and GQA groups 1, 4 and 16."""
+ends inside a tile, split key ranges, and GQA groups 1, 4 and 16. And ticks of
+GQA groups 1 and 2 whose waves end far apart."""
 
 import math
 
 import pytest
 import torch
+
+from test_prefill_ring import FAR
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +72,40 @@ def test_rows_off_sixteen_bytes(hq, hkv, cache, q_len, shift):
         want = torch.softmax(s.masked_fill(mask, -math.inf), -1) @ v[head // grp]
         err = (outs[0][:, head].float() - want).norm() / want.norm()
         assert err < 1e-2, float(err)  # bf16 probabilities and output
+
+
+@pytest.mark.parametrize("group,cache,q_lens", FAR)
+def test_waves_that_end_tiles_apart(group, cache, q_lens):
+    """Few heads a group: a workgroup's waves span up to 256 tokens, and an early
+    one's last V block must not be gone when it multiplies it."""
+    hkv = 8
+    g = torch.Generator(device="cuda").manual_seed(group + sum(q_lens))
+    m = PagedKVCacheManager(1, hkv, 128, 16_384, 128, len(cache), torch.bfloat16, "cuda",
+                            num_q_heads=hkv * group)
+    m.k_cache.normal_(generator=g)
+    m.v_cache.normal_(generator=g)
+    handles = []
+    for c in cache:
+        h = m.allocate()
+        m.reserve(h, c)
+        h.length = c
+        handles.append(h)
+    batch = m.begin_tick(handles, q_lens)
+    q = torch.randn(sum(q_lens), hkv * group, 128, generator=g, device="cuda").to(torch.bfloat16)
+    outs = [batch.attend_layer(q, 0).clone() for _ in range(3)]
+    row = 0
+    for h, c, n in zip(handles, cache, q_lens):
+        t = torch.arange(c + n, device="cuda")
+        where = torch.tensor(h.pages, device="cuda")[t // 128] * 128 + t % 128
+        k = m.k_cache[0, 0][:, where].float().repeat_interleave(group, 0)
+        v = m.v_cache[0, 0][:, where].float().repeat_interleave(group, 0)
+        late = t[None] > (c + torch.arange(n, device="cuda"))[:, None]
+        s = (q[row : row + n].float().transpose(0, 1) @ k.transpose(1, 2).contiguous()) / math.sqrt(128)
+        want = (torch.softmax(s.masked_fill(late, -math.inf), -1) @ v).transpose(0, 1)
+        for out in outs:
+            got = out[row : row + n].float()
+            # row by row: a wave holds 32 of them
+            err = (got - want).norm(dim=-1) / want.norm(dim=-1)
+            assert err.max() < 3e-2, float(err.max())  # bf16 probabilities and output
+        row += n
+    assert all(torch.equal(o.view(torch.int16), outs[0].view(torch.int16)) for o in outs)
