@@ -42,8 +42,11 @@ def _views_of(f: torch.Tensor, ws) -> bool:
 
 
 def _norm_eps(norm: nn.RMSNorm, dtype: torch.dtype) -> float:
-    """The epsilon nn.RMSNorm applies to inputs of `dtype`."""
-    return float(norm.eps) if norm.eps is not None else float(torch.finfo(dtype).eps)
+    """The epsilon nn.RMSNorm applies to inputs of `dtype`: its default is that
+    of the type it computes in, fp32 for 16-bit inputs."""
+    if norm.eps is not None:
+        return float(norm.eps)
+    return torch.finfo(torch.float64 if dtype is torch.float64 else torch.float32).eps
 
 
 class GroupedQueryAttention(nn.Module):
@@ -133,8 +136,7 @@ class GroupedQueryAttention(nn.Module):
         B, T = q.shape[:2]
         q_norm, k_norm = self.q_norm, self.k_norm
         q_norm_w, k_norm_w = q_norm.weight, k_norm.weight
-        # each norm keeps its own eps; None means the input dtype's epsilon,
-        # as nn.RMSNorm resolves it
+        # each norm keeps its own eps; None is resolved as nn.RMSNorm does
         eps = _norm_eps(q_norm, q.dtype)
         k_eps = _norm_eps(k_norm, k.dtype)
         if paged_cache.varlen:

@@ -187,3 +187,28 @@ def test_head_of_a_tick():
         hook.remove()
     assert logits.shape == plain.shape == (3, 1, 1000)
     assert rel(logits, plain.double()) < 2**-7
+
+
+@pytest.mark.parametrize("tokens", [3, 40])
+def test_norms_without_an_epsilon(tokens):
+    """eps=None is the module's default also on the fused paths: rows of rms
+    0.05, which another epsilon would change by more than the roundings."""
+    cfg = Qwen3Config(hidden_size=1024, num_heads=8, num_kv_groups=2, intermediate_size=2048,
+                      vocab_size=1000, num_layers=1, rms_norm_eps=None)
+    with torch.device(DEV):
+        model = Qwen3Model(cfg)
+    init_synthetic_weights(model, 4)
+    with torch.no_grad():
+        model.embed_tokens.weight.normal_(std=0.05)
+        for w in (model.layers[0].self_attn.o_proj, model.layers[0].mlp.down_proj):
+            w.weight.mul_(0.01)  # the rows stay small up to the head
+    ids = torch.arange(tokens, device=DEV).view(1, tokens)
+    _, batch = tick(cfg, [tokens - 2, 1, 1])
+    with torch.inference_mode():
+        logits = model(ids, paged_cache=batch)[0]
+        hooks = [m.register_forward_hook(lambda *a: None)
+                 for m in (model.norm, model.layers[0].mlp)]
+        plain = model(ids, paged_cache=batch)[0]
+        for h in hooks:
+            h.remove()
+    assert rel(logits, plain.double()) < 2**-7

@@ -1,9 +1,10 @@
 """Host-side pieces of the attention module and model that run without a
 GPU: the fused q/k/v projection and the checkpoint name map."""
 
+import pytest
 import torch
 
-from hayate_amd.attention import GroupedQueryAttention
+from hayate_amd.attention import GroupedQueryAttention, _norm_eps
 from hayate_amd.model import Qwen3Config, Qwen3Model, qwen_weight_map
 
 
@@ -91,3 +92,17 @@ def test_stop_ids_from_generation_config_and_tokenizer(tmp_path):
     assert _stop_token_ids(str(tmp_path), tok) == {7}
     assert _stop_token_ids(None, tok) == {7}
     assert _stop_token_ids(str(tmp_path / "missing"), None) == set()
+
+
+@pytest.mark.parametrize("eps", [None, 0.0, 1e-6, 0.25])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32, torch.float64])
+def test_norm_epsilon_is_the_modules(dtype, eps):
+    """Rows small enough for the epsilon to decide the result."""
+    g = torch.Generator().manual_seed(0)
+    norm = torch.nn.RMSNorm(256, eps=eps, dtype=dtype)
+    x = (torch.randn(8, 256, generator=g) * 1e-3).to(dtype)
+    e = _norm_eps(norm, dtype)
+    want = x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + e)
+    # one rounding of the result; fp32 sums add far less
+    tol = torch.finfo(dtype).eps if dtype is not torch.float64 else 1e-12
+    assert ((norm(x).double() - want).norm() / want.norm()) < max(tol, 1e-6 * (tol > 1e-12))
