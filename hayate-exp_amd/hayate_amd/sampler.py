@@ -110,7 +110,10 @@ def _sample_native(logits, temperature, top_k, top_p, generator):
     dev = logits.device
     temp = np.asarray(temperature, dtype=np.float32)
     k = np.asarray([vocab if v is None else min(v, vocab) for v in top_k], dtype=np.int32)
+    # a top_p that fp32 rounds to 0 keeps what the smallest number does: the
+    # logits with no mass before them
     p = np.asarray([1.0 if v is None else v for v in top_p], dtype=np.float32)
+    p = np.maximum(p, np.finfo(np.float32).tiny)
     drawn = int(np.count_nonzero(temp))
     noise = valid = None
     if drawn:

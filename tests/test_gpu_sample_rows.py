@@ -107,6 +107,22 @@ def test_masked_and_extreme_rows():
     assert out.flatten().tolist() == [40, 50, 20]
 
 
+@pytest.mark.parametrize("p", [5e-324, 1e-50, 7e-46, 1e-38, 1e-30])
+def test_smallest_top_p(p):
+    """Down to the smallest positive double: the first of the largest logits."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    x = torch.randn(4, 3000, generator=g, device=DEV).to(torch.bfloat16)
+    x[0, [700, 40, 2999]] = 9.0
+    first = (x == x.max(1, keepdim=True).values).int().argmax(1).tolist()
+    assert first[0] == 40
+    args = [1.0, 0.5, 2.0, 0.0], [None, 50, None, None], [p, p, p, 1e-50]
+    out = sample_batch(x, *args, torch.Generator(device=DEV).manual_seed(1))
+    assert out.flatten().tolist() == first
+    # the sorted path, whose sort may leave equal scores in any order
+    out = sample_batch(x.float(), *args, torch.Generator(device=DEV).manual_seed(1))
+    assert torch.equal(x.gather(1, out), x.max(1, keepdim=True).values)
+
+
 def test_rows_without_a_distribution_are_reported():
     """*valid through the C ABI: a NaN, only -inf, +inf; sample_batch turns it
     into an error as torch.multinomial does."""
