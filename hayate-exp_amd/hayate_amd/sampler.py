@@ -92,15 +92,17 @@ MAX_VOCAB = 4_194_304
 
 def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
     """True when hy_sample takes these rows: 16-bit logits on the current HIP
-    device, contiguous along the vocabulary, temperatures whose scores keep
-    the logits' order (outside [1e-30, 1e30] they vanish or overflow and become
-    equal), and nothing watching the ops."""
+    device, contiguous along the vocabulary, whole numbers as top_k (the path
+    below refuses others), temperatures whose scores keep the logits' order
+    (outside [1e-30, 1e30] they vanish or overflow and become equal), and
+    nothing watching the ops."""
     return (type(logits) is torch.Tensor and logits.dtype in _DTYPES and logits.is_cuda
             and logits.dim() == 2 and logits.shape[0] > 0 and 0 < logits.shape[1] <= MAX_VOCAB
             and logits.stride(1) == 1
             and len(temperature) == len(top_k) == len(top_p) == logits.shape[0]
             and all(t == 0 or 1e-30 <= t <= 1e30 for t in temperature)
-            and all(k is None or k >= 1 for k in top_k)
+            and all(k is None or (type(k) is int or isinstance(k, np.integer)) and k >= 1
+                    for k in top_k)
             and all(p is None or p > 0 for p in top_p)
             and linear.unwatched() and logits.device.index == torch.cuda.current_device())
 
@@ -108,11 +110,11 @@ def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
 def _sample_native(logits, temperature, top_k, top_p, generator):
     n, vocab = logits.shape
     dev = logits.device
-    temp = np.asarray(temperature, dtype=np.float32)
+    temp = np.asarray([float(t) for t in temperature], dtype=np.float32)
     k = np.asarray([vocab if v is None else min(v, vocab) for v in top_k], dtype=np.int32)
     # a top_p that fp32 rounds to 0 keeps what the smallest number does: the
     # logits with no mass before them
-    p = np.asarray([1.0 if v is None else v for v in top_p], dtype=np.float32)
+    p = np.asarray([1.0 if v is None else float(v) for v in top_p], dtype=np.float32)
     p = np.maximum(p, np.finfo(np.float32).tiny)
     drawn = int(np.count_nonzero(temp))
     noise = valid = None

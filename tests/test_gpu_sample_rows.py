@@ -11,6 +11,7 @@ if both tokens are kept by a float64 cut with that slack.
 
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -121,6 +122,26 @@ def test_smallest_top_p(p):
     # the sorted path, whose sort may leave equal scores in any order
     out = sample_batch(x.float(), *args, torch.Generator(device=DEV).manual_seed(1))
     assert torch.equal(x.gather(1, out), x.max(1, keepdim=True).values)
+
+
+def test_parameter_types():
+    """Settings held in tensors and arrays as in Python numbers; a fractional
+    top_k is refused for 16-bit logits as for 32-bit ones."""
+    g = torch.Generator(device=DEV).manual_seed(10)
+    x = torch.randn(3, 3000, generator=g, device=DEV).to(torch.bfloat16)
+
+    def draw(t, k, p):
+        return sample_batch(x, t, k, p, torch.Generator(device=DEV).manual_seed(2)).tolist()
+
+    want = draw([0.5, 0.0, 2.0], [20, None, 7], [0.75, None, 0.5])
+    temp, p = torch.tensor([0.5, 0.0, 2.0]), torch.tensor([0.75, 1.0, 0.5])
+    for dev in ("cpu", DEV):
+        assert draw(temp.to(dev), [20, None, 7], p.to(dev)) == want
+        assert draw(list(temp.to(dev)), [20, None, torch.tensor(7, device=dev)], list(p)) == want
+    assert draw(temp.numpy(), np.array([20, 3000, 7]), p.numpy()) == want
+    for logits in (x, x.float()):
+        with pytest.raises((RuntimeError, TypeError)):
+            sample_batch(logits, [0.5, 0.0, 2.0], [20.5, None, 7], [None] * 3)
 
 
 def test_rows_without_a_distribution_are_reported():
