@@ -259,10 +259,13 @@ __global__ __launch_bounds__(kCutThreads) void cut_kernel(
     finish();
     return;
   }
-  // exp(score - max), in the exp2 domain
-  const float slope = rcp * kLog2eS, offset = -mx * kLog2eS;
+  // exp(score - max), in the exp2 domain. The logits are subtracted before they
+  // are scaled: of score * log2(e) and max * log2(e) the roundings alone are
+  // hundreds apart at a temperature of 1e-8, and one fma of the two would leave
+  // infinite or no mass.
+  const float slope = rcp * kLog2eS, top_value = value_of<kBf16>(top_key);
   auto mass_of = [&](uint32_t key) __attribute__((always_inline)) {
-    return __builtin_amdgcn_exp2f(__builtin_fmaf(value_of<kBf16>(key), slope, offset));
+    return __builtin_amdgcn_exp2f((value_of<kBf16>(key) - top_value) * slope);
   };
 
   // `wide`: 32-bit counters of the keys of one half (bit 15 `held`) at a time.

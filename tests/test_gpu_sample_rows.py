@@ -124,6 +124,32 @@ def test_smallest_top_p(p):
     assert torch.equal(x.gather(1, out), x.max(1, keepdim=True).values)
 
 
+@pytest.mark.parametrize("t", [1e-30, 1e-20, 1e-9, 1e-8, 1e-7, 1e-4, 1e4, 1e30])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_small_and_large_temperatures(t, dtype):
+    """Scores of up to 4e31: ties at the maximum are cut by index as at any
+    temperature. Below 1e-4 the maximum has all the mass (its neighbour is 1/64
+    of it away or more, 150 in the exponent), in equal parts."""
+    g = torch.Generator(device=DEV).manual_seed(11)
+    for top in (4.0, 17.25, 40.0):
+        x = (torch.rand(8, 20_000, generator=g, device=DEV) * 3.5).to(getattr(torch, dtype))
+        ties = [5, 800, 801, 9000, 19_999]
+        x[:, ties] = top
+        p = [0.1, 0.3, 0.39, 0.5, 0.7, 0.81, 0.99, 1.0]
+        seen = [set() for _ in p]
+        for seed in range(60):
+            out = sample_batch(x, [t] * 8, [None] * 8, p,
+                               torch.Generator(device=DEV).manual_seed(seed))
+            for s, i in zip(seen, out.flatten().tolist()):
+                s.add(i)
+        if t <= 1e-4:
+            # logit j of the five stays while the mass before it, j / 5, is within p
+            want = [set(ties[: 1 + sum(j / 5 <= q for j in range(1, 5))]) for q in p]
+            assert seen == want, (t, top)
+        if t < 1e4:  # (beyond, all logits weigh the same, which the rounding of
+            check(x, 1)  # 20,000 sums moves the cuts of)
+
+
 def test_parameter_types():
     """Settings held in tensors and arrays as in Python numbers; a fractional
     top_k is refused for 16-bit logits as for 32-bit ones."""
