@@ -88,6 +88,7 @@ def sample_batch(logits: torch.Tensor, temperature: Sequence[float],
 
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
 MAX_VOCAB = 4_194_304
+_TINY = float(np.finfo(np.float32).tiny)
 
 
 def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
@@ -110,12 +111,11 @@ def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
 def _sample_native(logits, temperature, top_k, top_p, generator):
     n, vocab = logits.shape
     dev = logits.device
-    temp = np.asarray([float(t) for t in temperature], dtype=np.float32)
+    temp = np.asarray(list(map(float, temperature)), dtype=np.float32)
     k = np.asarray([vocab if v is None else min(v, vocab) for v in top_k], dtype=np.int32)
     # a top_p that fp32 rounds to 0 keeps what the smallest number does: the
     # logits with no mass before them
-    p = np.asarray([1.0 if v is None else float(v) for v in top_p], dtype=np.float32)
-    p = np.maximum(p, np.finfo(np.float32).tiny)
+    p = np.asarray([1.0 if v is None else max(float(v), _TINY) for v in top_p], dtype=np.float32)
     drawn = int(np.count_nonzero(temp))
     noise = valid = None
     if drawn:
