@@ -13,17 +13,36 @@ leave the modules in charge.
 
 from __future__ import annotations
 
+import sys
 from typing import Optional
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 from torch.nn.modules import module as _module
 
 from . import _native
 
 MAX_ROWS = 32
 _MAX_STRIDE = 1 << 22
-_Parameter, _Linear, _RMSNorm = nn.Parameter, nn.Linear, nn.RMSNorm
+_BF16 = torch.bfloat16
+_Parameter, _Module, _Linear, _RMSNorm = nn.Parameter, nn.Module, nn.Linear, nn.RMSNorm
+
+
+def _as_shipped(f, home) -> object:
+    """`f` if it is the function that module `home` defines, else an object that
+    nothing compares equal to: patched before this import, it stays in charge."""
+    code = getattr(f, "__code__", None)
+    return f if code is not None and code.co_filename == home.__file__ else object()
+
+
+# What calling a module and the functions in it runs, unless somebody has put
+# something else in their place.
+_CALL = _as_shipped(nn.Module.__call__, _module)
+_LINEAR = _as_shipped(nn.Linear.forward, sys.modules["torch.nn.modules.linear"])
+_NORM = _as_shipped(nn.RMSNorm.forward, sys.modules["torch.nn.modules.normalization"])
+_F_LINEAR = torch._C._nn.linear
+_RMS_NORM, _SILU = _as_shipped(F.rms_norm, F), _as_shipped(F.silu, F)
 
 
 def unwatched() -> bool:
@@ -51,27 +70,35 @@ def few_rows(x: torch.Tensor) -> bool:
     return takes(x) and x.numel() <= MAX_ROWS * x.shape[-1]
 
 
+def _unpatched() -> bool:
+    """True when calling the modules of a block runs torch's own code."""
+    return (_Module.__call__ is _CALL and _Linear.forward is _LINEAR and _Linear.__call__ is _CALL
+            and _RMSNorm.forward is _NORM and _RMSNorm.__call__ is _CALL
+            and F.linear is _F_LINEAR and F.rms_norm is _RMS_NORM and F.silu is _SILU)
+
+
 def _bare(m: nn.Module) -> bool:
-    """No hooks and no forward of its own."""
+    """No hooks and no forward of its own, compiled or not."""
     d = m.__dict__
     return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
-                or d["_backward_pre_hooks"] or "forward" in d)
+                or d["_backward_pre_hooks"] or "forward" in d or "_compiled_call_impl" in d)
 
 
 def _plain_weight(w, device_index: int, dim: int) -> bool:
-    if (type(w) is not _Parameter or w.dtype is not torch.bfloat16
+    if (type(w) is not _Parameter or w.dtype is not _BF16 or w.data_ptr() & 15
             or w.get_device() != device_index):
         return False
     st = w.stride()
-    return (len(st) == dim and st[-1] == 1 and w.data_ptr() & 15 == 0
-            and (dim == 1 or (st[0] & 7 == 0 and st[0] < _MAX_STRIDE)))
+    if dim == 1:
+        return st == (1,)
+    return len(st) == 2 and st[1] == 1 and st[0] & 7 == 0 and st[0] < _MAX_STRIDE
 
 
 def plain(x: torch.Tensor, modules=(), norms=(), linears=()) -> bool:
     """True when calling `modules`, `norms` (over x's last dimension) and
     `linears` would do nothing but their own arithmetic on weights that the
     kernels can read."""
-    if _module._has_any_global_hook():
+    if _module._has_any_global_hook() or not _unpatched():
         return False
     index, shape = x.get_device(), (x.shape[-1],)
     for m in modules:
@@ -84,7 +111,7 @@ def plain(x: torch.Tensor, modules=(), norms=(), linears=()) -> bool:
     for m in linears:
         if type(m) is not _Linear or not _bare(m):
             return False
-        p = m._parameters
+        p = m.__dict__["_parameters"]
         if p.get("bias") is not None or not _plain_weight(p.get("weight"), index, 2):
             return False
     return True

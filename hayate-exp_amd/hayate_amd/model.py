@@ -44,6 +44,12 @@ class Qwen3Config:
     max_position_embeddings: int = 40_960
 
 
+# Methods that the fused paths below stand in for; a replaced one, of the class
+# or of an instance, is left in charge.
+_ATTENTION_FORWARD = GroupedQueryAttention.forward
+_PROJECT_QKV = GroupedQueryAttention.project_qkv
+
+
 class _Weights(NamedTuple):
     """What a block's fused paths read (the q, k and v weights are the
     attention module's fused buffer)."""
@@ -67,6 +73,9 @@ class FeedForward(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.down_proj(nn.functional.silu(self.gate_proj(x)) * self.up_proj(x))
+
+
+_MLP_FORWARD = FeedForward.forward
 
 
 class TransformerBlock(nn.Module):
@@ -108,7 +117,10 @@ class TransformerBlock(nn.Module):
         modules would, else None."""
         mods = self._modules
         attn, mlp = mods.get("self_attn"), mods.get("mlp")
-        if type(attn) is not GroupedQueryAttention or type(mlp) is not FeedForward or x.dim() != 3:
+        if (type(attn) is not GroupedQueryAttention or type(mlp) is not FeedForward or x.dim() != 3
+                or GroupedQueryAttention.forward is not _ATTENTION_FORWARD
+                or GroupedQueryAttention.project_qkv is not _PROJECT_QKV
+                or "project_qkv" in attn.__dict__ or FeedForward.forward is not _MLP_FORWARD):
             return None
         # straight from the modules' tables: nn.Module's attribute lookup takes
         # about 0.5 us a name, and this runs for every layer of every tick

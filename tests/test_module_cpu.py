@@ -4,8 +4,10 @@ GPU: the fused q/k/v projection and the checkpoint name map."""
 import pytest
 import torch
 
+from hayate_amd import linear
 from hayate_amd.attention import GroupedQueryAttention, _norm_eps
-from hayate_amd.model import Qwen3Config, Qwen3Model, qwen_weight_map
+from hayate_amd.model import (FeedForward, Qwen3Config, Qwen3Model, TransformerBlock,
+                              qwen_weight_map)
 
 
 def test_fused_qkv_projection_views_one_gemm():
@@ -106,3 +108,65 @@ def test_norm_epsilon_is_the_modules(dtype, eps):
     # one rounding of the result; fp32 sums add far less
     tol = torch.finfo(dtype).eps if dtype is not torch.float64 else 1e-12
     assert ((norm(x).double() - want).norm() / want.norm()) < max(tol, 1e-6 * (tol > 1e-12))
+
+
+@pytest.fixture
+def plain_block(monkeypatch):
+    """A block whose weights the fused paths would take if they were on the GPU."""
+    monkeypatch.setattr(linear, "_plain_weight", lambda w, index, dim: True)
+    cfg = Qwen3Config(hidden_size=64, num_heads=4, num_kv_groups=2, head_dim=16,
+                      intermediate_size=96, vocab_size=50, num_layers=1)
+    block = TransformerBlock(cfg)
+    x = torch.zeros(1, 3, 64, dtype=torch.bfloat16)
+    assert block._plain_weights(x) is not None
+    return block, x
+
+
+def _keep(f):
+    return lambda *a, **k: f(*a, **k)
+
+
+@pytest.mark.parametrize("owner,name", [
+    (torch.nn.Linear, "forward"), (torch.nn.Linear, "__call__"), (torch.nn.RMSNorm, "forward"),
+    (torch.nn.RMSNorm, "__call__"), (torch.nn.Module, "__call__"),
+    (torch.nn.functional, "linear"), (torch.nn.functional, "rms_norm"),
+    (torch.nn.functional, "silu"), (FeedForward, "forward"), (GroupedQueryAttention, "forward"),
+    (GroupedQueryAttention, "project_qkv")])
+def test_replaced_functions_stay_in_charge(plain_block, monkeypatch, owner, name):
+    block, x = plain_block
+    with monkeypatch.context() as m:
+        m.setattr(owner, name, _keep(getattr(owner, name)), raising=True)
+        assert block._plain_weights(x) is None
+    assert block._plain_weights(x) is not None
+
+
+@pytest.mark.parametrize("path,name", [
+    ("self_attn", "forward"), ("self_attn", "project_qkv"), ("mlp", "forward"),
+    ("mlp.up_proj", "forward"), ("self_attn.o_proj", "forward"), ("input_layernorm", "forward"),
+    ("post_attention_layernorm", "forward")])
+def test_an_instances_own_method_stays_in_charge(plain_block, path, name):
+    block, x = plain_block
+    m = block.get_submodule(path)
+    setattr(m, name, _keep(getattr(m, name)))
+    assert block._plain_weights(x) is None
+    delattr(m, name)
+    assert block._plain_weights(x) is not None
+    m.compile(backend="eager")
+    assert block._plain_weights(x) is None
+
+
+def test_functions_replaced_before_the_import_stay_in_charge():
+    code = """
+import torch
+F = torch.nn.functional
+real, torch.nn.Linear.forward = torch.nn.Linear.forward, lambda self, x: real(self, x)
+from hayate_amd import linear
+assert not linear._unpatched()
+torch.nn.Linear.forward = real
+"""
+    import os
+    import subprocess
+    import sys
+
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path))
+    subprocess.run([sys.executable, "-c", code], check=True, env=env, timeout=300)
