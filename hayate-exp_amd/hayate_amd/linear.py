@@ -19,13 +19,16 @@ from typing import Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad as _forward_ad
 from torch.nn.modules import module as _module
+from torch.utils._device import DeviceContext as _DeviceContext
 
 from . import _native
 
 MAX_ROWS = 32
 _MAX_STRIDE = 1 << 22
 _BF16 = torch.bfloat16
+_C, _peek_functorch = torch._C, torch._C._functorch.peek_interpreter_stack
 _Parameter, _Module, _Linear, _RMSNorm = nn.Parameter, nn.Module, nn.Linear, nn.RMSNorm
 
 
@@ -41,18 +44,22 @@ def _as_shipped(f, home) -> object:
 _CALL = _as_shipped(nn.Module.__call__, _module)
 _LINEAR = _as_shipped(nn.Linear.forward, sys.modules["torch.nn.modules.linear"])
 _NORM = _as_shipped(nn.RMSNorm.forward, sys.modules["torch.nn.modules.normalization"])
-_F_LINEAR = torch._C._nn.linear
+_F_LINEAR = _C._nn.linear
 _RMS_NORM, _SILU = _as_shipped(F.rms_norm, F), _as_shipped(F.silu, F)
 
 
 def unwatched() -> bool:
     """True when nothing watches the operators a call runs: tracing, dispatch or
-    function modes, functorch, forward-mode gradients."""
-    c = torch._C
-    return (c._len_torch_dispatch_stack() == 0 and c._len_torch_function_stack() == 0
-            and c._get_tracing_state() is None and not torch.compiler.is_compiling()
-            and torch.autograd.forward_ad._current_level < 0
-            and c._functorch.peek_interpreter_stack() is None)
+    function modes, functorch, forward-mode gradients. A default device is held
+    in a function mode too, but watches nothing: it names the device of factory
+    calls that leave theirs open, which the callers of this do not."""
+    n = _C._len_torch_function_stack()
+    return (_C._len_torch_dispatch_stack() == 0
+            and (n == 0 or all(type(_C._get_function_stack_at(i)) is _DeviceContext
+                               for i in range(n)))
+            and _C._get_tracing_state() is None and not torch.compiler.is_compiling()
+            and _forward_ad._current_level < 0
+            and _peek_functorch() is None)
 
 
 def takes(x: torch.Tensor) -> bool:

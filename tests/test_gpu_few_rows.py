@@ -212,3 +212,42 @@ def test_norms_without_an_epsilon(tokens):
         for h in hooks:
             h.remove()
     assert rel(logits, plain.double()) < 2**-7
+
+
+@pytest.mark.parametrize("device", ["cpu", "cuda", "meta"])
+@pytest.mark.parametrize("tokens", [4, 70])
+def test_a_default_device_keeps_the_kernels(device, tokens, monkeypatch):
+    """Logits and tokens under torch.device(...): the same bits by the same
+    kernels."""
+    from hayate_amd import _native
+    from hayate_amd.sampler import sample_batch
+
+    cfg = Qwen3Config(hidden_size=512, num_heads=8, num_kv_groups=2, intermediate_size=1024,
+                      vocab_size=1000, num_layers=1)
+    with torch.device(DEV):
+        model = Qwen3Model(cfg)
+    init_synthetic_weights(model, 6)
+    model.initialize_rope(DEV)
+    ids = torch.arange(tokens, device=DEV).view(1, tokens)
+
+    def call():
+        _, batch = tick(cfg, [tokens - 2, 1, 1])
+        batch.plan(cfg.num_heads)
+        used = []
+        for name in ("norm_linear", "linear_add", "row_norm", "tile_linear"):
+            real = getattr(linear, name)
+            monkeypatch.setattr(linear, name,
+                                lambda *a, f=real, n=name, **k: (used.append(n), f(*a, **k))[1])
+        with torch.inference_mode():
+            logits = model(ids, paged_cache=batch)[0]
+            tokens_ = sample_batch(logits[:, 0], [0.0, 0.7, 1.0], [None, 20, None],
+                                   [None, None, 0.9], torch.Generator(device=DEV).manual_seed(3))
+        monkeypatch.undo()
+        return logits, tokens_, used
+
+    want = call()
+    assert set(want[2]) == ({"norm_linear", "linear_add"} if tokens < 32 else
+                            {"row_norm", "tile_linear", "norm_linear"})
+    with torch.device(device):
+        got = call()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and got[2] == want[2]

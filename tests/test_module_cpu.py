@@ -170,3 +170,28 @@ torch.nn.Linear.forward = real
 
     env = dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path))
     subprocess.run([sys.executable, "-c", code], check=True, env=env, timeout=300)
+
+
+def test_a_default_device_watches_nothing():
+    from torch.overrides import TorchFunctionMode
+
+    class Watcher(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert linear.unwatched()
+    for device in ("cpu", "meta", "cuda"):
+        with torch.device(device):
+            assert linear.unwatched()
+            with Watcher():
+                assert not linear.unwatched()
+            with torch.device("cpu"):
+                assert linear.unwatched()
+        with Watcher(), torch.device(device):
+            assert not linear.unwatched()
+        try:
+            torch.set_default_device(device)
+            assert linear.unwatched()
+        finally:
+            torch.set_default_device(None)
+    assert linear.unwatched()
