@@ -126,8 +126,10 @@ __device__ __forceinline__ void load_to_lds(const uint16_t *g, const uint16_t *l
   const uint32_t m0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
       (const __attribute__((address_space(3))) uint16_t *)lds));
   // M0 has no other user in this kernel (no LDS-DMA builtins, no indexed
-  // register access), so setting it here disturbs nothing.
-  __asm__ volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+  // register access), so setting it here disturbs nothing. A load that reads M0
+  // must not directly follow its write: the ISA asks for one wait state, which
+  // the compiler does not add inside an assembly block.
+  __asm__ volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                    :
                    : "v"(g), "s"(__builtin_amdgcn_readfirstlane(m0))
                    : "memory");
