@@ -137,12 +137,16 @@ void wide_kernel(const uint16_t *__restrict__ x, int64_t ldx, int m_rows, int k_
   issue(a1, min(c0 + kTile, c1 - 1));
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) turn(b[mt]);
+  auto drop_others = [&]() {  // steps that another wave owns
+    if (own == 0) return;
 #pragma unroll
-  for (int s = 0; s < SPW; ++s)
-    if (s < own) {
+    for (int s = 0; s < SPW; ++s)
+      if (s < own) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) b[mt][s] = u32x4{0u, 0u, 0u, 0u};
-    }
+        for (int mt = 0; mt < MT; ++mt) b[mt][s] = u32x4{0u, 0u, 0u, 0u};
+      }
+  };
+  drop_others();
 
   if (norm_w != nullptr) {
     // Row sums of squares over this wave's k: the diagonal of x x^T, whose
@@ -171,6 +175,7 @@ void wide_kernel(const uint16_t *__restrict__ x, int64_t ldx, int m_rows, int k_
         b[mt][s] = pack8_rne(v);
       }
     }
+    drop_others();  // again: no 0 * inf of an infinite weight
   }
 
   // Output (m, n) of a tile: thread m * kTile + n, the same for every tile.

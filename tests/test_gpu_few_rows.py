@@ -94,6 +94,18 @@ def test_infinite_weights_stay_in_their_columns():
     assert not torch.isnan(y).any()
 
 
+@pytest.mark.parametrize("at", [0, 447, 448, 470, 575])
+def test_infinite_norm_weights(at):
+    """An infinite norm weight gives the infinities it gives torch's norm and
+    product, no NaN, also where the waves' windows overlap (from 448 on)."""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    x, w, nw = bf16(g, 5, 576), bf16(g, 64, 576), 1 + bf16(g, 576, std=0.1)
+    nw[at] = float("inf")
+    x[:, at], w[:, at] = x[:, at].abs() + 0.1, w[:, at].abs() + 0.1
+    y = linear.norm_linear(x, nw, 1e-6, w)
+    assert (y == float("inf")).all()
+
+
 def tick(cfg, q_lens, layers=1):
     m = PagedKVCacheManager(layers, cfg.num_kv_groups, cfg.head_dim, 32_768, 128, len(q_lens),
                             torch.bfloat16, DEV, num_q_heads=cfg.num_heads)
