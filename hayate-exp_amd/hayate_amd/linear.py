@@ -79,8 +79,8 @@ def few_rows(x: torch.Tensor) -> bool:
 
 def _unpatched() -> bool:
     """True when calling the modules of a block runs torch's own code."""
-    return (_Module.__call__ is _CALL and _Linear.forward is _LINEAR and _Linear.__call__ is _CALL
-            and _RMSNorm.forward is _NORM and _RMSNorm.__call__ is _CALL
+    return (_Linear.__call__ is _CALL and _RMSNorm.__call__ is _CALL and _Module.__call__ is _CALL
+            and _Linear.forward is _LINEAR and _RMSNorm.forward is _NORM
             and F.linear is _F_LINEAR and F.rms_norm is _RMS_NORM and F.silu is _SILU)
 
 
@@ -134,23 +134,32 @@ def add_fits(k: int, rows: int) -> bool:
     return k % 128 == 0 and k > 0 and rows <= MAX_ROWS
 
 
-def tiles_fit(k: int, n: int, rows: int) -> bool:
-    """Sizes hy_linear_tiles takes (the kernels' rows are at most _MAX_STRIDE
-    apart, which rows_of sees to for x)."""
-    return (k % 64 == 0 and n % 4 == 0 and 0 < k < _MAX_STRIDE
-            and (rows // 64 + 1) * (n // 48 + 1) < 1 << 23)
+def tiles_fit(d: int, heads: int, mid: int, rows: int) -> bool:
+    """Sizes hy_row_norm and hy_linear_tiles take for a block of d inputs, `heads`
+    values of attention and `mid` of the MLP (x's rows are at most _MAX_STRIDE
+    apart, which rows_of sees to)."""
+    n = d if d > mid else mid
+    return ((d | heads | mid) % 64 == 0 and 0 < d <= 4096 and 0 < heads < _MAX_STRIDE
+            and 0 < mid < _MAX_STRIDE and (rows // 64 + 1) * (n // 48 + 1) < 1 << 23)
 
 
-def row_norm_fits(k: int) -> bool:
-    """Sizes hy_row_norm takes."""
-    return k % 8 == 0 and 0 < k <= 4096
+def tiles_add_pays(k: int, n: int, rows: int) -> bool:
+    """Whether hy_linear_tiles with a residual keeps up with the library's product
+    and addition. Its tiles and their split of k are for outputs that do not fill
+    the chip; on many the library's kernels are ahead. Measured on MI355X over n =
+    1024 .. 4096 and k = n .. 4 n (time over the library's, by millions of outputs):
+    below 4 0.75-1.1, mean 0.95; 4 to 5.5 0.91-1.15, mean 1.03; 6 to 9 1.05; 13 to
+    16 up to 1.33 (9728 -> 2560, 512 rows 35 / 47 us, 2064 109 / 111, 6000 283 /
+    215). With a very long k the library falls behind for longer (25600 -> 5120:
+    1700 rows 0.63, 2064 1.31)."""
+    return rows * n <= (11 << 19 if k <= 16_384 else 1 << 23)
 
 
 def rows_of(x: torch.Tensor) -> torch.Tensor:
     """x (..., d) as (rows, d) with rows the kernels can read."""
     x = x.reshape(-1, x.shape[-1])
-    if (x.stride(1) != 1 or x.stride(0) & 7 or x.stride(0) >= _MAX_STRIDE
-            or x.data_ptr() & 15):
+    row, one = x.stride()
+    if one != 1 or row & 7 or row >= _MAX_STRIDE or x.data_ptr() & 15:
         x = x.contiguous()
         if x.data_ptr() & 15:
             x = x.clone()

@@ -101,8 +101,7 @@ class TransformerBlock(nn.Module):
                 if (linear.norm_fits(d, rows) and linear.add_fits(heads, rows)
                         and linear.add_fits(mid, rows)):
                     return self._few_rows(x, w, cos, sin, paged_cache, layer_idx), None, None
-                if (linear.row_norm_fits(d) and linear.tiles_fit(heads, d, rows)
-                        and linear.tiles_fit(d, mid, rows) and linear.tiles_fit(mid, d, rows)):
+                if linear.tiles_fit(d, heads, mid, rows):
                     return self._many_rows(x, w, cos, sin, paged_cache, layer_idx), None, None
         shortcut = x
         x, new_k, new_v = self.self_attn(self.input_layernorm(x), cos, sin, position_ids, prev_k,
@@ -130,11 +129,11 @@ class TransformerBlock(nn.Module):
                    f.get("gate_proj"), f.get("up_proj"), f.get("down_proj")]
         if not linear.plain(x, modules=(attn, mlp), norms=norms, linears=linears):
             return None
-        q, k, v, o, gate, up, down = [m._parameters["weight"] for m in linears]
+        q, _, _, o, gate, up, down = [m.__dict__["_parameters"]["weight"] for m in linears]
         d, heads, shape = x.shape[2], attn.num_heads * attn.head_dim, gate.shape
-        if (q.shape != (heads, d) or k.shape[1] != d or v.shape[1] != d or o.shape != (d, heads)
-                or shape[1] != d or up.shape != shape or up.stride() != gate.stride()
-                or down.shape != (d, shape[0])):
+        # k and v have q's columns, or the fused q/k/v buffer cannot be built
+        if (q.shape != (heads, d) or o.shape != (d, heads) or shape[1] != d or up.shape != shape
+                or up.stride() != gate.stride() or down.shape != (d, shape[0])):
             return None
         return _Weights(in_norm, post_norm, o, gate, up, down)
 
@@ -154,17 +153,23 @@ class TransformerBlock(nn.Module):
         return linear.linear_add(h, w.down, x).view(shape)
 
     def _many_rows(self, x, w, cos, sin, paged_cache, layer_idx):
-        """The block for a prompt's rows: silu, the gating product and the
-        residuals inside the products. The q/k/v projection has nothing to
-        fuse and stays with the library."""
+        """The block for a prompt's rows: silu, the gating product and, up to some
+        size, the residuals inside the products. The q/k/v projection has nothing
+        to fuse and stays with the library."""
         attn, shape = self._modules["self_attn"], x.shape
         x = linear.rows_of(x)
         h = linear.row_norm(x, w.in_norm._parameters["weight"], _norm_eps(w.in_norm, x.dtype))
         context = attn.context(*attn.project_qkv(h.view(shape)), cos, sin, paged_cache, layer_idx)
-        x = linear.tile_linear(linear.rows_of(context), w.o, residual=x)
+        rows, d = x.shape
+        if linear.tiles_add_pays(context.shape[-1], d, rows):
+            x = linear.tile_linear(linear.rows_of(context), w.o, residual=x)
+        else:
+            x = nn.functional.linear(context.view(-1, context.shape[-1]), w.o).add_(x)
         h = linear.row_norm(x, w.post_norm._parameters["weight"], _norm_eps(w.post_norm, x.dtype))
         h = linear.tile_linear(h, w.gate, w.up)
-        return linear.tile_linear(h, w.down, residual=x).view(shape)
+        if linear.tiles_add_pays(h.shape[1], d, rows):
+            return linear.tile_linear(h, w.down, residual=x).view(shape)
+        return nn.functional.linear(h, w.down).add_(x).view(shape)
 
 
 class Qwen3Model(nn.Module):

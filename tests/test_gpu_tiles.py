@@ -126,3 +126,36 @@ def test_block_equals_its_modules(lens):
             hook.remove()
     # five roundings of 2^-8 in a chain of products at most
     assert rel(outs[0], outs[1].double()) < 5 * 2**-8
+
+
+@pytest.mark.parametrize("rows,tiles", [(33, 3), (11_264, 3), (11_265, 1), (13_000, 1)])
+def test_many_outputs_leave_the_residual_products_to_the_library(rows, tiles, monkeypatch):
+    """On both sides of the line (rows x 512 outputs): how many products take the
+    tiles, and the block against its modules."""
+    cfg = Qwen3Config(hidden_size=512, num_heads=8, num_kv_groups=8, intermediate_size=512)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    with torch.device(DEV):
+        block = TransformerBlock(cfg).eval()
+    with torch.no_grad():
+        for p in block.parameters():
+            p.copy_(bf16(g, *p.shape, std=p.shape[-1] ** -0.5) if p.dim() == 2 else 1 + bf16(g, *p.shape, std=0.1))
+    lens = [512] * (rows // 512) + [rows % 512] * (rows % 512 > 0)
+    x = bf16(g, 1, rows, 512)
+    cos = torch.randn(1024, 128, generator=g, device=DEV)
+    sin = torch.randn(1024, 128, generator=g, device=DEV)
+    used = []
+    real = linear.tile_linear
+    monkeypatch.setattr(linear, "tile_linear", lambda *a, **k: (used.append(1), real(*a, **k))[1])
+    outs = []
+    for hooked in (False, True):
+        mgr = PagedKVCacheManager(1, 8, 128, 32_768, 128, len(lens), torch.bfloat16, DEV, num_q_heads=8)
+        batch = mgr.begin_tick([mgr.allocate() for _ in lens], lens)
+        hook = block.mlp.register_forward_hook(lambda *a: None) if hooked else None
+        before = x.clone()
+        with torch.no_grad():
+            outs.append(block(x, cos, sin, None, None, None, None, batch, 0)[0])
+        if hook:
+            hook.remove()
+        assert torch.equal(x, before)
+    assert len(used) == tiles
+    assert rel(outs[0], outs[1].double()) < 5 * 2**-8  # five roundings in a chain at most
