@@ -91,12 +91,22 @@ MAX_VOCAB = 4_194_304
 _TINY = float(np.finfo(np.float32).tiny)
 
 
+def _greedy_pays(rows: int, vocab: int) -> bool:
+    """Whether hy_sample beats torch.argmax where every row is greedy: one
+    workgroup a row against a reduction that is slow on a few long rows only, and
+    splits a single row past 131,072 values. Measured on MI355X (us, hy_sample /
+    argmax): 20 rows of 151,936 17 / 38, 128 of them 32 / 48, 256 53 / 49; 20 of
+    65,536 16 / 19, 64 of them 22 / 20; 20 of 32,000 17 / 12; one of 151,936 14 / 12,
+    of 100,352 14 / 26."""
+    return vocab >= 65_536 and rows * 1400 <= vocab and (rows > 1 or vocab <= 131_072)
+
+
 def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
     """True when hy_sample takes these rows: 16-bit logits on the current HIP
     device, contiguous along the vocabulary, whole numbers as top_k (the path
     below refuses others), temperatures whose scores keep the logits' order
-    (outside [1e-30, 1e30] they vanish or overflow and become equal), and
-    nothing watching the ops."""
+    (outside [1e-30, 1e30] they vanish or overflow and become equal), nothing
+    watching the ops, and not only greedy rows that argmax is faster for."""
     return (type(logits) is torch.Tensor and logits.dtype in _DTYPES and logits.is_cuda
             and logits.dim() == 2 and logits.shape[0] > 0 and 0 < logits.shape[1] <= MAX_VOCAB
             and logits.stride(1) == 1
@@ -105,6 +115,7 @@ def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
             and all(k is None or (type(k) is int or isinstance(k, np.integer)) and k >= 1
                     for k in top_k)
             and all(p is None or p > 0 for p in top_p)
+            and (any(t != 0 for t in temperature) or _greedy_pays(*logits.shape))
             and linear.unwatched() and logits.device.index == torch.cuda.current_device())
 
 

@@ -150,6 +150,29 @@ def test_small_and_large_temperatures(t, dtype):
             check(x, 1)  # 20,000 sums moves the cuts of)
 
 
+@pytest.mark.parametrize("n,vocab,native", [
+    (1, 9, 0), (1, 65_536, 1), (1, 131_072, 1), (1, 131_073, 0), (2, 65_535, 0), (46, 65_536, 1),
+    (47, 65_536, 0), (108, 151_936, 1), (109, 151_936, 0), (300, 1000, 0)])
+def test_greedy_batches(n, vocab, native, monkeypatch):
+    """All rows greedy, on both sides of the line between hy_sample and argmax; one
+    row with a temperature and the whole batch is hy_sample's."""
+    from hayate_amd import sampler
+
+    used = []
+    real = sampler._sample_native
+    monkeypatch.setattr(sampler, "_sample_native", lambda *a: (used.append(1), real(*a))[1])
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn(n, vocab, generator=g, device=DEV).to(torch.bfloat16)
+    x[:, vocab // 2], x[0, 3] = 9.0, math.nan
+    want = [3] + [vocab // 2] * (n - 1)
+    out = sample_batch(x, [0.0] * n, [None] * n, [0.5] * n)
+    assert out.flatten().tolist() == want and len(used) == native
+    x[0, 3] = 0.0
+    out = sample_batch(x, [1.0] + [0.0] * (n - 1), [1] + [None] * (n - 1), [None] * n,
+                       torch.Generator(device=DEV).manual_seed(1))
+    assert out.flatten().tolist() == [vocab // 2] * n and len(used) == native + 1
+
+
 def test_parameter_types():
     """Settings held in tensors and arrays as in Python numbers; a fractional
     top_k is refused for 16-bit logits as for 32-bit ones."""
