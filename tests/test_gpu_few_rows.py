@@ -125,7 +125,7 @@ def tick(cfg, q_lens, layers=1):
 def test_block_equals_its_modules(q_lens, monkeypatch):
     """The fused block against the same block with a hook on its MLP (which
     puts the modules back in charge): both within the block's rounding of
-    each other; 33 rows take the modules either way."""
+    each other; 33 rows take the tile products instead of the few-row ones."""
     say(f"[block, q_lens {q_lens}]")
     cfg = Qwen3Config()
     torch.manual_seed(3)
@@ -142,6 +142,9 @@ def test_block_equals_its_modules(q_lens, monkeypatch):
     used = []
     real = linear.linear_add
     monkeypatch.setattr(linear, "linear_add", lambda *a: (used.append(1), real(*a))[1])
+    tiles = []
+    tile = linear.tile_linear
+    monkeypatch.setattr(linear, "tile_linear", lambda *a, **k: (tiles.append(1), tile(*a, **k))[1])
     m, batch = tick(cfg, q_lens)
     with torch.inference_mode():
         fused = block(x, cos, sin, None, None, None, None, batch, 0)[0]
@@ -151,6 +154,7 @@ def test_block_equals_its_modules(q_lens, monkeypatch):
         plain = block(x, cos, sin, None, None, None, None, batch, 0)[0]
         hook.remove()
         assert len(used) == (2 if sum(q_lens) <= 32 else 0)
+        assert len(tiles) == (0 if sum(q_lens) <= 32 else 3)
     e = rel(fused, plain.double())
     say(f"  relative difference {e:.2e}")
     # five rounded products on either side, each 2^-8 of a part of the sum

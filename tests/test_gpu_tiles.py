@@ -1,16 +1,17 @@
 """The prompt-row products (csrc/tiles.hip) and the block that uses them.
 
-Against float64 at the sizes where the plan changes: every tile shape, split
-and whole, row and column counts that leave the last tile one row, all but
+Against float64: row and column counts that leave the last tile one row, all but
 one, or a fraction of a fragment, and K of one step, of fewer steps than the
-ring has stages and of many. The result is rounded to bf16 once (at most 2^-8
-of each value); the fp32 sums add far less.
+ring has stages and of many, on the small tiles; and every tile shape, split and
+whole, at sizes that test_tile_plan.py holds the plan to. The result is rounded
+to bf16 once (at most 2^-8 of each value); the fp32 sums add far less.
 """
 
 import pytest
 import torch
 
 from gpu_util import say
+from test_tile_plan import SIZES
 
 pytestmark = pytest.mark.gpu
 
@@ -57,6 +58,26 @@ def test_gated_linear(m, n, k):
     assert rel(linear.tile_linear(x, w, u), exact) < 2**-8
 
 
+@pytest.mark.parametrize("gated,m,n,k", SIZES)
+def test_every_plan(gated, m, n, k):
+    say(f"tiles plan {m} x {n} x {k}, gated {gated}")
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x, w = bf16(g, m, k), bf16(g, n, k, std=k**-0.5)
+    if gated:
+        u = bf16(g, n, k, std=k**-0.5)
+        gate = x.double() @ w.double().T
+        exact = gate * torch.sigmoid(gate) * (x.double() @ u.double().T)
+        assert rel(linear.tile_linear(x, w, u), exact) < 2**-8
+    else:
+        r = bf16(g, m, n)
+        exact = x.double() @ w.double().T + r.double()
+        y = linear.tile_linear(x, w, residual=r)
+        assert rel(y, exact) < 2**-8
+        # no single output is far off, which the norm would not show: the rounding,
+        # and fp32 sums of up to 5,824 terms (k 2^-24 sum|x w| < 2^-6 of them)
+        assert ((y.double() - exact).abs() <= 2**-8 * exact.abs() + 2**-6).all()
+
+
 @pytest.mark.parametrize("k", [8, 504, 512, 520, 2560, 3592, 4096])
 @pytest.mark.parametrize("m", [1, 33, 4096, 4099])
 def test_row_norm(m, k):
@@ -99,10 +120,14 @@ def test_infinities_and_nans_stay_in_their_rows():
 
 
 @pytest.mark.parametrize("lens", [(40,), (256, 1, 44), (600,)])
-def test_block_equals_its_modules(lens):
+def test_block_equals_its_modules(lens, monkeypatch):
     """The fused block against the modules' own calls (taken when a hook is
     there), both bf16: each output is within the roundings of the fused one's
     fewer intermediates."""
+    used = []
+    for name in ("tile_linear", "row_norm"):
+        monkeypatch.setattr(linear, name, lambda *a, f=getattr(linear, name), n=name, **k:
+                            (used.append(n), f(*a, **k))[1])
     cfg = Qwen3Config(hidden_size=1024, num_heads=16, num_kv_groups=8, intermediate_size=3072)
     g = torch.Generator(device=DEV).manual_seed(sum(lens))
     with torch.device(DEV):
@@ -124,6 +149,8 @@ def test_block_equals_its_modules(lens):
             outs.append(block(x, cos, sin, None, None, None, None, batch, 0)[0])
         if hook:
             hook.remove()
+        # by the fused block only
+        assert used.count("tile_linear") == 3 and used.count("row_norm") == 2
     # five roundings of 2^-8 in a chain of products at most
     assert rel(outs[0], outs[1].double()) < 5 * 2**-8
 
