@@ -115,7 +115,7 @@ def _native_rows(logits: torch.Tensor, temperature, top_k, top_p) -> bool:
             and all(k is None or (type(k) is int or isinstance(k, np.integer)) and k >= 1
                     for k in top_k)
             and all(p is None or p > 0 for p in top_p)
-            and (any(t != 0 for t in temperature) or _greedy_pays(*logits.shape))
+            and (any(temperature) or _greedy_pays(*logits.shape))
             and linear.unwatched() and logits.device.index == torch.cuda.current_device())
 
 
@@ -140,7 +140,7 @@ def _sample_native(logits, temperature, top_k, top_p, generator):
         logits.data_ptr(), logits.stride(0), _DTYPES[logits.dtype], n, vocab, temp.ctypes.data,
         k.ctypes.data, p.ctypes.data, noise.data_ptr() if drawn else None, out.data_ptr(),
         valid.data_ptr() if drawn else None, work.data_ptr(), work.numel(),
-        torch.cuda.current_stream(dev).cuda_stream)
+        _native.stream_of(logits.get_device()))
     if rc:
         _native.check(rc, "hy_sample")
     if drawn:
