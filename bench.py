@@ -482,7 +482,7 @@ def main():
 
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) > 1:
         print("bench.py measures one GPU only: the paged-attention path runs on one "
-              "MI355X; multi-GPU runs are not part of this build.", file=sys.stderr)
+              "MI355X; multi-GPU runs are not supported.", file=sys.stderr)
         sys.exit(2)
     if not torch.cuda.is_available():
         print("bench.py needs a HIP GPU", file=sys.stderr)

@@ -515,7 +515,7 @@ void prefill_kernel(
   s_a = qk();
   read_k(1);
 
-  // Tile t: tile t + 2's loads go into the stage tile t - 1 used (every wave
+  // Tile t: tile t + 2's loads go into the stage tile t - 2 used (every wave
   // left it before the last barrier), then this wave's blocks 2t, 2t + 1;
   // the barrier publishes tile t + 2, which the K reads two blocks ahead
   // need during tile t + 1. A block body always runs the next block's

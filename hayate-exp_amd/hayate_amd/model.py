@@ -164,7 +164,7 @@ class TransformerBlock(nn.Module):
         if linear.tiles_add_pays(context.shape[-1], d, rows):
             x = linear.tile_linear(linear.rows_of(context), w.o, residual=x)
         else:
-            x = nn.functional.linear(context.view(-1, context.shape[-1]), w.o).add_(x)
+            x = nn.functional.linear(context.reshape(rows, -1), w.o).add_(x)
         h = linear.row_norm(x, w.post_norm._parameters["weight"], _norm_eps(w.post_norm, x.dtype))
         h = linear.tile_linear(h, w.gate, w.up)
         if linear.tiles_add_pays(h.shape[1], d, rows):

@@ -1,6 +1,6 @@
 """CPU restatement of the reference's paged-attention path.
 
-TEST INFRASTRUCTURE ONLY. This module is the checker: only tests/,
+TEST INFRASTRUCTURE ONLY. This module is the oracle: only tests/,
 __graft_entry__.smoke() and bench.py's cpu_baseline leg may import it, and
 only to compute expected values or a reported CPU timing. The product path
 (hayate-exp_amd/hayate_amd) never imports it.
